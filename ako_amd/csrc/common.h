@@ -141,15 +141,20 @@ __device__ __forceinline__ float dpp_mov(float v) {
       float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-  v += dpp_mov<0xB1>(v);   // quad_perm [1,0,3,2]: lane ^ 1
-  v += dpp_mov<0x4E>(v);   // quad_perm [2,3,0,1]: lane ^ 2
-  v += dpp_mov<0x141>(v);  // row_half_mirror: the other quad of each 8 lanes
-  v += dpp_mov<0x140>(v);  // row_mirror: the other half of each 16-lane row
-  v += __shfl_xor(v, 16);
-  v += __shfl_xor(v, 32);
+// The same over each aligned group of L lanes (a power of two from 4 up).
+template <int L>
+__device__ __forceinline__ float lane_group_sum(float v) {
+  static_assert(L >= 4 && L <= kWave && (L & (L - 1)) == 0, "lanes per group");
+  v += dpp_mov<0xB1>(v);                            // quad_perm [1,0,3,2]: lane ^ 1
+  v += dpp_mov<0x4E>(v);                            // quad_perm [2,3,0,1]: lane ^ 2
+  if constexpr (L >= 8) v += dpp_mov<0x141>(v);     // row_half_mirror: the other quad of each 8 lanes
+  if constexpr (L >= 16) v += dpp_mov<0x140>(v);    // row_mirror: the other half of each 16-lane row
+  if constexpr (L >= 32) v += __shfl_xor(v, 16);
+  if constexpr (L >= 64) v += __shfl_xor(v, 32);
   return v;
 }
+
+__device__ __forceinline__ float wave_sum(float v) { return lane_group_sum<kWave>(v); }
 
 // ---- workgroup order over the XCDs ------------------------------------------
 // Workgroups are dispatched round-robin over the 8 XCDs (workgroup b runs on

@@ -1,6 +1,10 @@
 // RMSNorm and residual-add + RMSNorm for gfx950.
 //
-// Three kernels:
+// Four kernels:
+//
+// rmsnorm_short - rows of at most 64 packets (512 half-precision or 256 fp32
+//   elements: per-head norms): a row takes the 4-64 lanes that hold it, so a
+//   wavefront works on up to 16 rows at once.
 //
 // rmsnorm_reg  - the row lives in registers. A row is owned by WPR wavefronts
 //   (64 * WPR lanes); lane t of the row holds the 16-byte packets
@@ -10,8 +14,7 @@
 //   residual) written once, all with the non-temporal hint; the weight row
 //   is re-read by every row and stays in L2. The sum of squares is reduced
 //   in fp32 with DPP inside the wavefront and, when WPR > 1, through WPR
-//   floats of LDS. Small rows pack RPB rows into one workgroup (the decode
-//   shapes: 1 or 32 rows). A lane issues every load of a group of packets
+//   floats of LDS. Small rows pack RPB rows into one workgroup. A lane issues every load of a group of packets
 //   before consuming any of them, so its memory latency is paid once per
 //   group instead of once per packet. Wide rows are handed to the 8 XCDs in
 //   runs of consecutive rows (block_order) rather than row by row.
@@ -45,6 +48,8 @@
 namespace ako {
 
 RmsTuning g_rms_tuning;
+
+constexpr int kShortBlock = 256;  // lanes per workgroup of rmsnorm_short
 
 // E elements of the weight row held as raw packets (one 16-byte packet, or
 // two when the weight is fp32 and the input half precision).
@@ -219,6 +224,85 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void rmsnorm_reg(
     }
   }
   if (has_tail) yr[tcol] = from_f32<T>((to_f32(vt) * rstd) * to_f32(w[tcol]));
+}
+
+// rmsnorm_short - a row of at most L packets is owned by L lanes (4-64, a power
+// of two), lane j holding packet j, so one wavefront-wide load covers 64 / L
+// whole rows: dense rows stream 1 KiB per instruction whatever their width. A
+// workgroup of 256 lanes takes U groups of 256 / L consecutive rows. The sum
+// of squares needs no LDS: the butterfly of wave_sum over the row's own lanes,
+// in the same order, so the sums are bitwise those of a whole wavefront per
+// row with its spare lanes at zero.
+//
+// Bound by memory. One wavefront per row (rmsnorm_reg (1, 1)) left 64 - nvec
+// lanes of every load idle. MI355X, bf16, 2^25 elements, cold, against that:
+// rows of 128: plain 55.8 -> 22.7 us (5.9 TB/s), residual 74.8 -> 43.4 us
+// (6.2 TB/s); rows of 32: 185 -> 22.8 us; rows of 256: 33.4 -> 22.6 us; rows of
+// 512: 24.5 -> 22.6 us. Decode-sized launches: 256 rows of 128 1.79 -> 1.77 us.
+template <typename T, typename W, int L, int U, bool RES>
+__global__ __launch_bounds__(kShortBlock) void rmsnorm_short(
+    const T* __restrict__ x, const T* __restrict__ res, const W* __restrict__ w, T* __restrict__ y,
+    T* __restrict__ rout, int64_t row0, int64_t rows, int hidden, int64_t sx, int64_t sr, int64_t sy,
+    int64_t srout, float inv_h, float eps) {
+  constexpr int E = 16 / static_cast<int>(sizeof(T));
+  constexpr int R = kShortBlock / L;  // rows per group
+  using P = Pack<T, E>;
+  const int j = threadIdx.x % L;
+  const int nvec = hidden / E;
+  const int tail = hidden - nvec * E;
+  const int64_t first = row0 + static_cast<int64_t>(blockIdx.x) * (R * U) + threadIdx.x / L;
+  const bool has_packet = j < nvec;
+  const bool has_tail = j < tail;  // the launcher gives L >= tail lanes
+  P v[U];
+  [[maybe_unused]] P rv[U];
+  T vt[U];
+  [[maybe_unused]] T rt[U];
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    const int64_t row = first + k * R;
+    if (row >= rows) continue;
+    if (has_packet) {
+      v[k] = load_pack<T, E, true>(x + row * sx + j * E);
+      if constexpr (RES) rv[k] = load_pack<T, E, true>(res + row * sr + j * E);
+    }
+    if (has_tail) {
+      vt[k] = x[row * sx + nvec * E + j];
+      if constexpr (RES) rt[k] = res[row * sr + nvec * E + j];
+    }
+  }
+  WeightPacket<W, E> wv;
+  if (has_packet) wv.load(w + j * E);
+#pragma unroll
+  for (int k = 0; k < U; ++k) {
+    const int64_t row = first + k * R;
+    const bool active = row < rows;
+    float ss = 0.f;
+    if (active && has_packet) {
+      if constexpr (RES) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[k].e[e] = from_f32<T>(to_f32(v[k].e[e]) + to_f32(rv[k].e[e]));
+        store_pack<T, E, true>(rout + row * srout + j * E, v[k]);
+      }
+      ss = sumsq_add(v[k], ss);
+    }
+    if (active && has_tail) {
+      if constexpr (RES) {
+        vt[k] = from_f32<T>(to_f32(vt[k]) + to_f32(rt[k]));
+        rout[row * srout + nvec * E + j] = vt[k];
+      }
+      const float f = to_f32(vt[k]);
+      ss = __builtin_fmaf(f, f, ss);
+    }
+    const float rstd = rsqrtf(lane_group_sum<L>(ss) * inv_h + eps);
+    if (active && has_packet) {
+      P o;
+#pragma unroll
+      for (int e = 0; e < E; ++e) o.e[e] = from_f32<T>((to_f32(v[k].e[e]) * rstd) * wv[e]);
+      store_pack<T, E, true>(y + row * sy + j * E, o);
+    }
+    if (active && has_tail)
+      y[row * sy + nvec * E + j] = from_f32<T>((to_f32(vt[k]) * rstd) * to_f32(w[nvec * E + j]));
+  }
 }
 
 // rmsnorm_pipe - rmsnorm_reg's row layout (WPR wavefronts per row, lane t
@@ -552,8 +636,8 @@ constexpr int kMaxRegPackets = 16 * 64 * 8;
 // per shape on MI355X, 16384 rows, fp16 and bf16: plain rows are fastest
 // with two packets per lane over 4-16 wavefronts; residual rows, which load
 // two tensors per packet, with one packet per lane over 8-16 wavefronts.
-// Rows that fit one wavefront's first packet stay on one wavefront so that
-// small rows need no LDS exchange and pack 4 rows per workgroup.
+// Rows of at most kShortPackets take rmsnorm_short before this, unless a
+// shape is forced.
 RegShape pick_shape(int64_t nvec, bool residual, int64_t rows) {
   // One packet per lane and more wavefronts per row for the residual variant,
   // and for plain rows when a launch has too few rows to give every CU a
@@ -828,10 +912,65 @@ hipError_t run_stream(const RmsArgs& a, hipStream_t stream) {
   return hipSuccess;
 }
 
+// Widest row (in packets) of rmsnorm_short.
+constexpr int kShortPackets = 64;
+
+template <typename T, typename W, int L, int U, bool RES>
+hipError_t run_short_groups(const RmsArgs& a, hipStream_t stream) {
+  constexpr int64_t per_block = kShortBlock / L * U;
+  const int64_t blocks = ceil_div(a.rows, per_block), cap = max_blocks_per_launch(kShortBlock);
+  for (int64_t b0 = 0; b0 < blocks; b0 += cap) {
+    const dim3 grid(static_cast<unsigned>(std::min(cap, blocks - b0)));
+    AKO_LAUNCH((rmsnorm_short<T, W, L, U, RES>), grid, dim3(kShortBlock), 0, stream, static_cast<const T*>(a.x),
+               static_cast<const T*>(a.r), static_cast<const W*>(a.w), static_cast<T*>(a.y),
+               static_cast<T*>(a.rout), b0 * per_block, a.rows, static_cast<int>(a.hidden), a.sx, a.sr, a.sy,
+               a.srout, 1.0f / static_cast<float>(a.hidden), a.eps);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) return err;
+  }
+  return hipSuccess;
+}
+
+// Row groups per workgroup: one, except for plain rows that leave lanes idle
+// (packets not a power of two) in launches of many workgroups, which take two
+// to have as many bytes in flight as full ones. MI355X, bf16, 2^25 elements,
+// one group against two: rows of 80 26.2 and 22.7 us, of 96 24.0 and 22.4, of
+// 192 24.2 and 22.3, but of 128 22.7 and 22.9; residual rows (two loads per
+// packet already) 43.4-44.2 and 44.4-45.0 at every width; 257 rows of 128 2.05
+// and 2.19 us.
+constexpr int64_t kShortTwoGroupBlocks = 4096;
+
+template <typename T, typename W, int L, bool RES>
+hipError_t run_short_lanes(const RmsArgs& a, hipStream_t stream) {
+  if constexpr (!RES) {
+    const bool idle_lanes = a.hidden < int64_t(L) * (16 / static_cast<int>(sizeof(T)));
+    if (idle_lanes && a.rows >= kShortTwoGroupBlocks * (kShortBlock / L))
+      return run_short_groups<T, W, L, 2, RES>(a, stream);
+  }
+  return run_short_groups<T, W, L, 1, RES>(a, stream);
+}
+
+// Lanes per row: the power of two that holds every packet, at least 8 (4 for
+// rows of whole packets), so that a partial packet's 1-7 elements have a lane
+// each.
+template <typename T, typename W, bool RES>
+hipError_t run_short(const RmsArgs& a, hipStream_t stream) {
+  constexpr int E = 16 / sizeof(T);
+  const int64_t nvec = a.hidden / E;
+  if (nvec <= 4 && nvec * E == a.hidden) return run_short_lanes<T, W, 4, RES>(a, stream);
+  if (nvec <= 8) return run_short_lanes<T, W, 8, RES>(a, stream);
+  if (nvec <= 16) return run_short_lanes<T, W, 16, RES>(a, stream);
+  if (nvec <= 32) return run_short_lanes<T, W, 32, RES>(a, stream);
+  return run_short_lanes<T, W, 64, RES>(a, stream);
+}
+
 template <typename T, typename W>
 hipError_t run_typed(const RmsArgs& a, hipStream_t stream) {
   constexpr int E = 16 / sizeof(T);
   const int64_t nvec = a.hidden / E;
+  const bool forced_shape = g_rms_tuning.waves_per_row > 0 || g_rms_tuning.vecs_per_thread > 0;
+  if (a.vector_ok && nvec <= kShortPackets && !forced_shape && g_rms_tuning.force_stream == 0)
+    return a.residual ? run_short<T, W, true>(a, stream) : run_short<T, W, false>(a, stream);
   const bool reg = a.vector_ok && g_rms_tuning.force_stream == 0 && nvec <= kMaxRegPackets &&
                    nvec >= 1;
   if (!reg) return a.residual ? run_stream<T, W, true>(a, stream) : run_stream<T, W, false>(a, stream);
@@ -849,7 +988,6 @@ hipError_t run_typed(const RmsArgs& a, hipStream_t stream) {
   // (512 or 2048 rows) they ran 7-15% slower than rmsnorm_reg, while
   // residual rows were as fast or faster from 300 rows up.
   const bool rows_ok = a.rows > kFewRows && a.rows < (int64_t(1) << 31) && nvec * E == a.hidden;
-  const bool forced_shape = g_rms_tuning.waves_per_row > 0 || g_rms_tuning.vecs_per_thread > 0;
   bool pipe = false;
   if (g_rms_tuning.pipeline == 2) {
     pipe = rows_ok && int64_t(s.wpr) * kWave * s.vpt == nvec && pipe_shape(s);
