@@ -234,12 +234,10 @@ static int rmsnorm_common(const void* x, const void* r, const void* w, void* y, 
         overlap(so_span, w_span) || overlap(so_span, sy_span))
       return fail(AKO_ERR_INVALID_ARGUMENT, "%s: residual_out overlaps another buffer", fn);
   }
-  bool vec = aligned(x, 16) && aligned(y, 16) && aligned(w, 16) && (sx * eb) % 16 == 0 &&
-             (sy * eb) % 16 == 0;
-  if (residual) vec = vec && aligned(r, 16) && aligned(rout, 16) && (sr * eb) % 16 == 0 && (srout * eb) % 16 == 0;
-  // Rows with a padded stride may be vector-aligned while hidden is not a
-  // multiple of the packet; the kernel handles that tail with scalar lanes.
-  ako::RmsArgs a{x, r, w, y, rout, rows, hidden, sx, sr, sy, srout, eps, dtype, w_dtype, residual, vec};
+  bool aligned16 = aligned(x, 16) && aligned(y, 16) && aligned(w, 16) && (sx * eb) % 16 == 0 && (sy * eb) % 16 == 0;
+  if (residual)
+    aligned16 = aligned16 && aligned(r, 16) && aligned(rout, 16) && (sr * eb) % 16 == 0 && (srout * eb) % 16 == 0;
+  ako::RmsArgs a{x, r, w, y, rout, rows, hidden, sx, sr, sy, srout, eps, dtype, w_dtype, residual, aligned16};
   return hip_status(ako::launch_rmsnorm(a, static_cast<hipStream_t>(stream)), fn);
 }
 
@@ -282,15 +280,12 @@ int ako_rmsnorm_shard_partial_fwd(const void* x, const void* residual, void* res
   const Span xs = span_2d(x, rows, shard, x_row_stride, eb);
   if (!ps.ok || !xs.ok) return fail(AKO_ERR_INVALID_ARGUMENT, "%s: sizes and strides overflow the address space", fn);
   if (shard > 0 && overlap(ps, xs)) return fail(AKO_ERR_INVALID_ARGUMENT, "%s: partial_ss overlaps x", fn);
-  bool vec = aligned(x, 16) && (x_row_stride * eb) % 16 == 0;
   if (res) {
     const Span rs = span_2d(residual, rows, shard, r_row_stride, eb);
     const Span os = span_2d(residual_out, rows, shard, rout_row_stride, eb);
     if (!rs.ok || !os.ok) return fail(AKO_ERR_INVALID_ARGUMENT, "%s: sizes and strides overflow the address space", fn);
     if (shard > 0 && (overlap(os, xs) || overlap(os, rs) || overlap(os, ps) || overlap(ps, rs)))
       return fail(AKO_ERR_INVALID_ARGUMENT, "%s: an output overlaps another buffer", fn);
-    vec = vec && aligned(residual, 16) && aligned(residual_out, 16) && (r_row_stride * eb) % 16 == 0 &&
-          (rout_row_stride * eb) % 16 == 0;
   }
   ako::RmsShardArgs a{};
   a.x = x;
@@ -304,7 +299,6 @@ int ako_rmsnorm_shard_partial_fwd(const void* x, const void* residual, void* res
   a.srout = rout_row_stride;
   a.dtype = dtype;
   a.residual = res;
-  a.vector_ok = vec;
   return hip_status(ako::launch_rmsnorm_shard_partial(a, static_cast<hipStream_t>(stream)), fn);
 }
 
@@ -336,8 +330,6 @@ int ako_rmsnorm_shard_apply_fwd(const void* s, const void* w, const float* total
     return fail(AKO_ERR_INVALID_ARGUMENT, "%s: sizes and strides overflow the address space", fn);
   if (overlap(ys, ss) || overlap(ys, ws) || overlap(ys, ts))
     return fail(AKO_ERR_INVALID_ARGUMENT, "%s: output y overlaps an input", fn);
-  const bool vec = aligned(s, 16) && aligned(y, 16) && aligned(w, 16) && (s_row_stride * eb) % 16 == 0 &&
-                   (y_row_stride * eb) % 16 == 0;
   ako::RmsShardArgs a{};
   a.x = s;
   a.w = w;
@@ -351,7 +343,6 @@ int ako_rmsnorm_shard_apply_fwd(const void* s, const void* w, const float* total
   a.eps = eps;
   a.dtype = dtype;
   a.w_dtype = w_dtype;
-  a.vector_ok = vec;
   return hip_status(ako::launch_rmsnorm_shard_apply(a, static_cast<hipStream_t>(stream)), fn);
 }
 

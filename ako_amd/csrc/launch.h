@@ -1,7 +1,7 @@
 // Internal launcher interface between the C ABI layer (abi.hip) and the
 // kernel translation units. Arguments reaching these functions have already
-// been validated by abi.hip: sizes positive, pointers non-null and aligned as
-// the chosen path requires, strides consistent.
+// been validated by abi.hip: sizes positive, pointers non-null, strides
+// consistent.
 #pragma once
 
 #include <hip/hip_ext.h>
@@ -95,7 +95,7 @@ struct RmsArgs {
   int dtype;
   int w_dtype;
   bool residual;
-  bool vector_ok;  // 16-byte packets are aligned for every row
+  bool aligned16;  // every tensor's rows start on 16-byte boundaries
 };
 hipError_t launch_rmsnorm(const RmsArgs& a, hipStream_t stream);
 
@@ -118,7 +118,6 @@ struct RmsShardArgs {
   int dtype;
   int w_dtype;
   bool residual;
-  bool vector_ok;
 };
 hipError_t launch_rmsnorm_shard_partial(const RmsShardArgs& a, hipStream_t stream);
 hipError_t launch_rmsnorm_shard_apply(const RmsShardArgs& a, hipStream_t stream);

@@ -24,12 +24,19 @@
 //   loads before it reduces and writes the current one. Taken by launches of
 //   many full rows of at most 16 KiB of input at one packet per lane.
 //
-// rmsnorm_stream - any width, any alignment (E = 1 scalar packets when the
-//   rows are not 16-byte aligned). One 256-lane workgroup per row, two passes
+// rmsnorm_stream - any width. One 256-lane workgroup per row, two passes
 //   over global memory: the first accumulates the sum of squares (and writes
 //   the rounded residual sum), the second re-reads and normalises. Used for
-//   rows wider than the register budget (> 65536 half-precision elements)
-//   and for misaligned rows.
+//   rows wider than the register budget (> 65536 half-precision elements).
+//
+// Rows may start at any element and have any width: packets need no alignment,
+// and the elements past a row's last whole packet take one lane each. Against
+// two passes in 2- or 4-byte accesses, MI355X, cold: fp16 rows of 4099, plain
+// 22.4 -> 9.8 us (2049 rows), 128 -> 55 us (16384 rows), residual 171 -> 109
+// us; one row 4.5 -> 1.9 us; fp32 rows of 2051, 16384 rows 89 -> 47 us. Half
+// rows at odd elements stay 15-25% behind aligned ones (2048 rows of 4096: 9.1
+// against 7.0 us; at multiples of two elements 7.0): a packet 2 bytes off a
+// dword takes the load path longer.
 //
 // Numerics follow the unfused reference (ako/ops/rmsnorm_ref.py:8-50):
 //   var  = sum(x^2) * (1/H)          (fp32; 1/H rounded to fp32 on the host)
@@ -86,7 +93,12 @@ __device__ __forceinline__ void store_write_through(T* row_base, int row_bytes, 
   __builtin_amdgcn_raw_buffer_store_b128(pk.raw, r, elem * static_cast<int>(sizeof(T)), 0, kStoreSc1Nt);
 }
 
-template <typename T, typename W, int WPR, int VPT, int RPB, bool RES, bool EW, bool SPLIT = false,
+// TAIL: rows end in a partial packet, whose elements take one lane each, requested
+// ahead of the packets so that they cost no round trip of their own. Rows of
+// whole packets are compiled without it: testing for a tail at run time, ahead
+// of the first loads or behind them, made wide whole-packet launches 0.4-2.5%
+// slower (16384 residual rows of 16384: 328 -> 330 and 336 us).
+template <typename T, typename W, int WPR, int VPT, int RPB, bool RES, bool EW, bool TAIL, bool SPLIT = false,
           bool WT = false>
 __global__ __launch_bounds__(kWave* WPR* RPB) void rmsnorm_reg(
     const T* __restrict__ x, const T* __restrict__ res, const W* __restrict__ w,
@@ -120,10 +132,19 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void rmsnorm_reg(
   const int64_t row = row0 + static_cast<int64_t>(block_order(blockIdx.x, gridDim.x, runs)) * RPB + row_in_block;
   const bool active = row < rows;
   const int nvec = hidden / E;
-  const int tail = hidden - nvec * E;
 
   const T* xr = x + row * sx;
   T* yr = y + row * sy;
+
+  [[maybe_unused]] T vt, rt;
+  [[maybe_unused]] const int tcol = nvec * E + t;
+  [[maybe_unused]] const bool has_tail = TAIL && active && tcol < hidden;
+  if constexpr (TAIL) {
+    if (has_tail) {
+      vt = xr[tcol];
+      if constexpr (RES) rt = res[row * sr + tcol];
+    }
+  }
 
   P v[VPT];
   WeightPacket<W, E> wv[G];
@@ -165,18 +186,15 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void rmsnorm_reg(
       }
     }
   }
-  // Elements past the last full packet (only when a row stride is padded).
-  T vt = from_f32<T>(0.f);
-  const int tcol = nvec * E + t;
-  const bool has_tail = active && t < tail;
-  if (has_tail) {
-    vt = xr[tcol];
-    if constexpr (RES) {
-      vt = from_f32<T>(to_f32(vt) + to_f32(res[row * sr + tcol]));
-      rout[row * srout + tcol] = vt;
+  if constexpr (TAIL) {
+    if (has_tail) {
+      if constexpr (RES) {
+        vt = from_f32<T>(to_f32(vt) + to_f32(rt));
+        rout[row * srout + tcol] = vt;
+      }
+      const float f = to_f32(vt);
+      ss = __builtin_fmaf(f, f, ss);
     }
-    const float f = to_f32(vt);
-    ss = __builtin_fmaf(f, f, ss);
   }
 
   // The weight row is L2-resident (every row reads it); fetch the first group
@@ -223,7 +241,9 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void rmsnorm_reg(
       }
     }
   }
-  if (has_tail) yr[tcol] = from_f32<T>((to_f32(vt) * rstd) * to_f32(w[tcol]));
+  if constexpr (TAIL) {
+    if (has_tail) yr[tcol] = from_f32<T>((to_f32(vt) * rstd) * to_f32(w[tcol]));
+  }
 }
 
 // rmsnorm_short - a row of at most L packets is owned by L lanes (4-64, a power
@@ -436,15 +456,15 @@ __global__ __launch_bounds__(kWave* WPR) void rmsnorm_pipe(
                                         srout, t, inv_h, eps);
 }
 
-// Two-pass kernel: one workgroup of kStreamBlock lanes per row, packets of E
-// elements (E = 16/sizeof(T) when aligned, else 1).
+// Two-pass kernel: one workgroup of kStreamBlock lanes per row.
 constexpr int kStreamBlock = 256;
 
-template <typename T, typename W, int E, bool RES>
+template <typename T, typename W, bool RES>
 __global__ __launch_bounds__(kStreamBlock) void rmsnorm_stream(
     const T* __restrict__ x, const T* __restrict__ res, const W* __restrict__ w,
     T* __restrict__ y, T* __restrict__ rout, int64_t row0, int hidden, int64_t sx, int64_t sr,
     int64_t sy, int64_t srout, float inv_h, float eps) {
+  constexpr int E = 16 / static_cast<int>(sizeof(T));
   using P = Pack<T, E>;
   const int64_t row = row0 + blockIdx.x;
   const int tid = threadIdx.x;
@@ -522,11 +542,12 @@ __global__ __launch_bounds__(kStreamBlock) void rmsnorm_stream(
 // ranks, and rmsnorm_shard_apply normalises each slice with the total:
 //   y = to_T((s * rsqrt(total * (1/H) + eps)) * w)
 // with H the full hidden size, the same arithmetic as rmsnorm_reg. One
-// 256-lane workgroup per row, packets of E elements (E = 1 when unaligned).
-template <typename T, int E, bool RES>
+// 256-lane workgroup per row.
+template <typename T, bool RES>
 __global__ __launch_bounds__(kStreamBlock) void rmsnorm_shard_partial(
     const T* __restrict__ x, const T* __restrict__ res, T* __restrict__ rout,
     float* __restrict__ partial, int64_t row0, int shard, int64_t sx, int64_t sr, int64_t srout) {
+  constexpr int E = 16 / static_cast<int>(sizeof(T));
   using P = Pack<T, E>;
   const int64_t row = row0 + blockIdx.x;
   const int tid = threadIdx.x;
@@ -543,7 +564,7 @@ __global__ __launch_bounds__(kStreamBlock) void rmsnorm_shard_partial(
     }
     ss = sumsq_add(p, ss);
   }
-  for (int j = nvec * E + tid; j < shard; j += kStreamBlock) {  // tail (E > 1 only)
+  for (int j = nvec * E + tid; j < shard; j += kStreamBlock) {  // past the last whole packet
     T v = xr[j];
     if constexpr (RES) {
       v = from_f32<T>(to_f32(v) + to_f32(res[row * sr + j]));
@@ -564,12 +585,13 @@ __global__ __launch_bounds__(kStreamBlock) void rmsnorm_shard_partial(
   }
 }
 
-template <typename T, typename W, int E, int R>
+template <typename T, typename W, int R>
 __global__ __launch_bounds__(kStreamBlock) void rmsnorm_shard_apply(
     const T* __restrict__ s, const W* __restrict__ w, const float* __restrict__ total,
     T* __restrict__ y, int64_t row0, int64_t rows, int shard, int64_t ss_, int64_t sy, float inv_h, float eps) {
   // Each workgroup applies R consecutive rows; a lane holds the same columns of
   // all R, so the weight packet is read once for R rows.
+  constexpr int E = 16 / static_cast<int>(sizeof(T));
   using P = Pack<T, E>;
   const int64_t first = row0 + static_cast<int64_t>(blockIdx.x) * R;
   const int tid = threadIdx.x;
@@ -696,7 +718,7 @@ int64_t max_blocks_per_launch(int threads_per_block) {
   return forced > 0 ? std::min(cap, forced) : cap;
 }
 
-template <typename T, typename W, int WPR, int VPT, bool RES, bool EW, bool SPLIT = false, bool WT = false>
+template <typename T, typename W, int WPR, int VPT, bool RES, bool EW, bool TAIL, bool SPLIT = false, bool WT = false>
 hipError_t run_reg_launch(const RmsArgs& a, hipStream_t stream) {
   constexpr int RPB = WPR >= 4 ? 1 : 4 / WPR;
   const dim3 block(kWave * WPR * RPB);
@@ -726,7 +748,7 @@ hipError_t run_reg_launch(const RmsArgs& a, hipStream_t stream) {
     const int order = g_rms_tuning.row_order, chunk = g_rms_tuning.xcd_chunk;
     if (order == 1) xcd_chunk = 1;
     if (order == 2) xcd_chunk = chunk > 0 ? unsigned(chunk) : unsigned(grid.x / 8);
-    AKO_LAUNCH((rmsnorm_reg<T, W, WPR, VPT, RPB, RES, EW, SPLIT, WT>),
+    AKO_LAUNCH((rmsnorm_reg<T, W, WPR, VPT, RPB, RES, EW, TAIL, SPLIT, WT>),
                grid, block, lds, stream, static_cast<const T*>(a.x), static_cast<const T*>(a.r),
                static_cast<const W*>(a.w), static_cast<T*>(a.y), static_cast<T*>(a.rout),
                b0 * RPB, a.rows, static_cast<int>(a.hidden), a.sx, a.sr, a.sy, a.srout,
@@ -751,13 +773,16 @@ constexpr int64_t kEarlyWeightRowBytes = 8 * 1024;
 
 template <typename T, typename W, int WPR, int VPT, bool RES>
 hipError_t run_reg(const RmsArgs& a, hipStream_t stream) {
+  const bool tail = a.hidden % (16 / static_cast<int>(sizeof(T))) != 0;
   if constexpr (VPT <= 2) {
     const int forced = g_rms_tuning.early_weights;
     const bool ew = forced == 2 ||
                     (forced == 0 && a.rows <= kFewRows &&
                      a.hidden * static_cast<int64_t>(sizeof(T)) <= kEarlyWeightRowBytes);
-    if (ew) return run_reg_launch<T, W, WPR, VPT, RES, true>(a, stream);
+    if (ew) return tail ? run_reg_launch<T, W, WPR, VPT, RES, true, true>(a, stream)
+                        : run_reg_launch<T, W, WPR, VPT, RES, true, false>(a, stream);
   }
+  if (tail) return run_reg_launch<T, W, WPR, VPT, RES, false, true>(a, stream);
   // Without write-through stores (key 12 = 1): one packet per load group for
   // bf16 residual rows of 16 wavefronts x 2 packets in launches of many rows.
   // Medians of 10 interleaved repetitions on MI355X, 16384 x 16384, cold
@@ -773,23 +798,25 @@ hipError_t run_reg(const RmsArgs& a, hipStream_t stream) {
   // of 8192, five buffer placements on each of three MI355X boxes, variants
   // interleaved, write-through was -0.43 to -0.55 points of peak for bf16
   // (every placement -0.17 or worse) and -0.33 to -0.42 for fp16. Key 12 = 2
-  // still selects it there.
+  // still selects it there. Buffer stores take whole aligned packets only:
+  // rows off a 16-byte boundary or with a partial packet store non-temporally.
   if constexpr ((VPT == 2 || VPT == 1) && WPR == 16) {
     constexpr bool kWtByDefault = VPT == 2;
     const int wt_forced = g_rms_tuning.write_through;
-    if (wt_forced == 2 || (wt_forced == 0 && kWtByDefault && a.rows > kFewRows)) {
+    if (a.aligned16 && (wt_forced == 2 || (wt_forced == 0 && kWtByDefault && a.rows > kFewRows))) {
       if constexpr (RES) {
-        if (g_rms_tuning.load_groups != 1) return run_reg_launch<T, W, WPR, VPT, RES, false, true, true>(a, stream);
+        if (g_rms_tuning.load_groups != 1)
+          return run_reg_launch<T, W, WPR, VPT, RES, false, false, true, true>(a, stream);
       }
-      return run_reg_launch<T, W, WPR, VPT, RES, false, false, true>(a, stream);
+      return run_reg_launch<T, W, WPR, VPT, RES, false, false, false, true>(a, stream);
     }
   }
   if constexpr (VPT == 2 && WPR == 16 && RES) {
     const int forced = g_rms_tuning.load_groups;
     const bool split = forced == 2 || (forced == 0 && std::is_same_v<T, __bf16> && a.rows > kFewRows);
-    if (split) return run_reg_launch<T, W, WPR, VPT, RES, false, true>(a, stream);
+    if (split) return run_reg_launch<T, W, WPR, VPT, RES, false, false, true>(a, stream);
   }
-  return run_reg_launch<T, W, WPR, VPT, RES, false>(a, stream);
+  return run_reg_launch<T, W, WPR, VPT, RES, false, false>(a, stream);
 }
 
 // Compute units of the current device (the pipelined grid's size), read
@@ -899,13 +926,8 @@ hipError_t run_stream(const RmsArgs& a, hipStream_t stream) {
   const int64_t cap = max_blocks_per_launch(kStreamBlock);
   for (int64_t r0 = 0; r0 < a.rows; r0 += cap) {
     const dim3 grid(static_cast<unsigned>(std::min(cap, a.rows - r0)));
-    if (a.vector_ok) {
-      AKO_LAUNCH((rmsnorm_stream<T, W, 16 / sizeof(T), RES>), grid, dim3(kStreamBlock), 0,
-                 stream, x, r, w, y, ro, r0, h, a.sx, a.sr, a.sy, a.srout, inv_h, a.eps);
-    } else {
-      AKO_LAUNCH((rmsnorm_stream<T, W, 1, RES>), grid, dim3(kStreamBlock), 0, stream, x, r,
-                 w, y, ro, r0, h, a.sx, a.sr, a.sy, a.srout, inv_h, a.eps);
-    }
+    AKO_LAUNCH((rmsnorm_stream<T, W, RES>), grid, dim3(kStreamBlock), 0, stream, x, r, w, y, ro, r0, h, a.sx,
+               a.sr, a.sy, a.srout, inv_h, a.eps);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
   }
@@ -969,10 +991,9 @@ hipError_t run_typed(const RmsArgs& a, hipStream_t stream) {
   constexpr int E = 16 / sizeof(T);
   const int64_t nvec = a.hidden / E;
   const bool forced_shape = g_rms_tuning.waves_per_row > 0 || g_rms_tuning.vecs_per_thread > 0;
-  if (a.vector_ok && nvec <= kShortPackets && !forced_shape && g_rms_tuning.force_stream == 0)
+  if (nvec <= kShortPackets && !forced_shape && g_rms_tuning.force_stream == 0)
     return a.residual ? run_short<T, W, true>(a, stream) : run_short<T, W, false>(a, stream);
-  const bool reg = a.vector_ok && g_rms_tuning.force_stream == 0 && nvec <= kMaxRegPackets &&
-                   nvec >= 1;
+  const bool reg = g_rms_tuning.force_stream == 0 && nvec <= kMaxRegPackets;
   if (!reg) return a.residual ? run_stream<T, W, true>(a, stream) : run_stream<T, W, false>(a, stream);
   RegShape s = pick_shape(nvec, a.residual, a.rows);
   // The pipelined kernel takes full rows only (no packet past the row's end)
@@ -1013,17 +1034,9 @@ hipError_t run_shard_partial(const RmsShardArgs& a, hipStream_t stream) {
   const int64_t cap = max_blocks_per_launch(kStreamBlock);
   for (int64_t r0 = 0; r0 < a.rows; r0 += cap) {
     const dim3 grid(static_cast<unsigned>(std::min(cap, a.rows - r0)));
-    if (a.vector_ok) {
-      AKO_LAUNCH((rmsnorm_shard_partial<T, 16 / sizeof(T), RES>), grid, dim3(kStreamBlock), 0,
-                 stream, static_cast<const T*>(a.x), static_cast<const T*>(a.r),
-                 static_cast<T*>(a.rout), a.partial, r0, static_cast<int>(a.shard), a.sx,
-                 a.sr, a.srout);
-    } else {
-      AKO_LAUNCH((rmsnorm_shard_partial<T, 1, RES>), grid, dim3(kStreamBlock), 0, stream,
-                 static_cast<const T*>(a.x), static_cast<const T*>(a.r),
-                 static_cast<T*>(a.rout), a.partial, r0, static_cast<int>(a.shard), a.sx,
-                 a.sr, a.srout);
-    }
+    AKO_LAUNCH((rmsnorm_shard_partial<T, RES>), grid, dim3(kStreamBlock), 0, stream,
+               static_cast<const T*>(a.x), static_cast<const T*>(a.r), static_cast<T*>(a.rout), a.partial, r0,
+               static_cast<int>(a.shard), a.sx, a.sr, a.srout);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
   }
@@ -1037,17 +1050,9 @@ hipError_t run_shard_apply_r(const RmsShardArgs& a, hipStream_t stream) {
   for (int64_t r0 = 0; r0 < a.rows; r0 += cap) {
     const int64_t end = std::min(a.rows, r0 + cap);
     const dim3 grid(static_cast<unsigned>(ceil_div(end - r0, R)));
-    if (a.vector_ok) {
-      AKO_LAUNCH((rmsnorm_shard_apply<T, W, 16 / sizeof(T), R>), grid, dim3(kStreamBlock), 0,
-                 stream, static_cast<const T*>(a.x), static_cast<const W*>(a.w), a.total,
-                 static_cast<T*>(a.y), r0, end, static_cast<int>(a.shard), a.sx, a.sy, inv_h,
-                 a.eps);
-    } else {
-      AKO_LAUNCH((rmsnorm_shard_apply<T, W, 1, R>), grid, dim3(kStreamBlock), 0, stream,
-                 static_cast<const T*>(a.x), static_cast<const W*>(a.w), a.total,
-                 static_cast<T*>(a.y), r0, end, static_cast<int>(a.shard), a.sx, a.sy, inv_h,
-                 a.eps);
-    }
+    AKO_LAUNCH((rmsnorm_shard_apply<T, W, R>), grid, dim3(kStreamBlock), 0, stream,
+               static_cast<const T*>(a.x), static_cast<const W*>(a.w), a.total, static_cast<T*>(a.y), r0, end,
+               static_cast<int>(a.shard), a.sx, a.sy, inv_h, a.eps);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
   }
