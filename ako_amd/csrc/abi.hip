@@ -570,11 +570,7 @@ int ako_swiglu_fwd(const void* gate, const void* up, void* y, int64_t rows, int6
   if (overlap(ys, gs) || overlap(ys, us))
     return fail(AKO_ERR_INVALID_ARGUMENT, "%s: output overlaps an input", fn);
   const bool contiguous = rows == 1 || (gate_row_stride == n && up_row_stride == n && y_row_stride == n);
-  const bool vec = aligned(gate, 16) && aligned(up, 16) && aligned(y, 16) &&
-                   (contiguous || ((gate_row_stride * eb) % 16 == 0 && (up_row_stride * eb) % 16 == 0 &&
-                                   (y_row_stride * eb) % 16 == 0));
-  ako::SwigluArgs a{gate, up, y, rows, n, gate_row_stride, up_row_stride, y_row_stride, dtype,
-                    contiguous, vec};
+  ako::SwigluArgs a{gate, up, y, rows, n, gate_row_stride, up_row_stride, y_row_stride, dtype, contiguous};
   return hip_status(ako::launch_swiglu(a, static_cast<hipStream_t>(stream)), fn);
 }
 

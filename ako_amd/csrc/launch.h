@@ -157,7 +157,6 @@ struct SwigluArgs {
   int64_t sg, su, sy;
   int dtype;
   bool contiguous;  // all three are one dense [rows * n] block
-  bool vector_ok;
 };
 hipError_t launch_swiglu(const SwigluArgs& a, hipStream_t stream);
 
