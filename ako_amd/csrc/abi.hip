@@ -184,7 +184,7 @@ int ako_set_tuning(int op, int key, int value) {
       }
       break;
     case 1:
-      if (key == 1) { ako::g_rope_tuning.tokens_per_block = value; return AKO_OK; }
+      if (key == 1) { ako::g_rope_tuning.waves_per_block = value; return AKO_OK; }
       if (key == 2) { ako::g_rope_tuning.iters = value; return AKO_OK; }
       if (key == 3) { ako::g_rope_tuning.xcd_chunk = value; return AKO_OK; }
       break;
@@ -458,20 +458,6 @@ int rope_common(const char* fn, const RopeTensorIn* ts, int nt, const void* cos,
     }
   }
 
-  const bool neox = style == AKO_ROPE_NEOX;
-  const int64_t E = 16 / eb;
-  const int64_t unit = neox ? head_dim / 2 : head_dim;
-  const int64_t table_vals = neox ? E : E / 2;  // table values one lane loads
-  const int64_t tab_align = std::min<int64_t>(16, table_vals * tb);
-  bool vec = unit % E == 0 && unit / E <= 64 && aligned(cos, tab_align) && aligned(sin, tab_align) &&
-             (st * tb) % tab_align == 0;
-  for (int i = 0; i < nt && vec; ++i) {
-    const RopeTensorIn& t = ts[i];
-    if (t.heads == 0) continue;
-    vec = aligned(t.x, 16) && aligned(t.y, 16);
-    for (int k = 0; k < 3 && vec; ++k) vec = t.xs[k] % E == 0 && t.ys[k] % E == 0;
-  }
-
   ako::RopeArgs a{};
   const ako::RopeTensorArgs none{nullptr, nullptr, 0, 0, 0, 0, 0, 0, 0};
   auto conv = [&](const RopeTensorIn& t) {
@@ -495,8 +481,7 @@ int rope_common(const char* fn, const RopeTensorIn* ts, int nt, const void* cos,
   a.st = st;
   a.dtype = dtype;
   a.table_dtype = table_dtype;
-  a.neox = neox;
-  a.vector_ok = vec;
+  a.neox = style == AKO_ROPE_NEOX;
   return hip_status(ako::launch_rope(a, static_cast<hipStream_t>(stream)), fn);
 }
 

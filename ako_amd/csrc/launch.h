@@ -70,9 +70,9 @@ struct RmsTuning {
   TuningKey write_through{0};    // key 12: (16, 2) and (16, 1) rows: 1 = non-temporal stores, 2 = write-through stores (0 = write-through on (16, 2) launches of many rows)
 };
 struct RopeTuning {
-  TuningKey tokens_per_block{0};  // key 1: wavefronts per workgroup (1, 2, 4, 8 or 16; one group per wavefront)
-  TuningKey iters{0};             // key 2: head chunks unrolled per loop trip
-  TuningKey xcd_chunk{0};         // key 3: consecutive workgroups per XCD run (1 = block order; 0 = runs of 128 for one tensor from 8192 workgroups)
+  TuningKey waves_per_block{0};  // key 1: wavefronts per workgroup (1, or 4 for any other value; 0 = by launch size)
+  TuningKey iters{0};            // key 2: accepted and unused (every lane moves one packet)
+  TuningKey xcd_chunk{0};        // key 3: consecutive workgroups per XCD run (1 = block order; 0 = by launch)
 };
 struct SwigluTuning {
   TuningKey vecs_per_thread{0};  // key 1: packets per lane (1, 2, 4 or 8)
@@ -145,7 +145,6 @@ struct RopeArgs {
   int64_t st;  // table row stride, elements
   int dtype, table_dtype;
   bool neox;
-  bool vector_ok;
 };
 hipError_t launch_rope(const RopeArgs& a, hipStream_t stream);
 
