@@ -98,8 +98,13 @@ __device__ __forceinline__ void store_write_through(T* row_base, int row_bytes, 
 // whole packets are compiled without it: testing for a tail at run time, ahead
 // of the first loads or behind them, made wide whole-packet launches 0.4-2.5%
 // slower (16384 residual rows of 16384: 328 -> 330 and 336 us).
-template <typename T, typename W, int WPR, int VPT, int RPB, bool RES, bool EW, bool TAIL, bool SPLIT = false,
-          bool WT = false>
+//
+// SUMS: separate sums of squares per lane, packet k going to sum k % SUMS and
+// each reduced on its own. A shape of WPR wavefronts then adds in the order of
+// one with SUMS * WPR wavefronts and 1 / SUMS of its packets per lane, so a
+// row's result does not depend on which of the two a launch takes.
+template <typename T, typename W, int WPR, int VPT, int RPB, bool RES, bool EW, bool TAIL, int SUMS = 1,
+          bool SPLIT = false, bool WT = false>
 __global__ __launch_bounds__(kWave* WPR* RPB) void rmsnorm_reg(
     const T* __restrict__ x, const T* __restrict__ res, const W* __restrict__ w,
     T* __restrict__ y, T* __restrict__ rout, int64_t row0, int64_t rows, int hidden, int64_t sx,
@@ -132,6 +137,11 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void rmsnorm_reg(
   const int64_t row = row0 + static_cast<int64_t>(block_order(blockIdx.x, gridDim.x, runs)) * RPB + row_in_block;
   const bool active = row < rows;
   const int nvec = hidden / E;
+  // Every argument is fetched here, in one scalar round trip; left alone the
+  // compiler fetches them in the branches around the loads and stores, one
+  // after another (1-8 rows of 2560-4096 half elements +0.06-0.08 us).
+  asm volatile("" : : "s"(x), "s"(w), "s"(sx), "s"(y), "s"(sy));
+  if constexpr (RES) asm volatile("" : : "s"(res), "s"(sr), "s"(rout), "s"(srout));
 
   const T* xr = x + row * sx;
   T* yr = y + row * sy;
@@ -148,7 +158,7 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void rmsnorm_reg(
 
   P v[VPT];
   WeightPacket<W, E> wv[G];
-  float ss = 0.f;
+  float ss[SUMS] = {};
 #pragma unroll
   for (int g0 = 0; g0 < VPT; g0 += G) {
     [[maybe_unused]] P rv[G];
@@ -182,7 +192,7 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void rmsnorm_reg(
           else
             store_pack<T, E, true>(rout + row * srout + vi * E, v[g0 + k]);
         }
-        ss = sumsq_add(v[g0 + k], ss);
+        ss[(g0 + k) % SUMS] = sumsq_add(v[g0 + k], ss[(g0 + k) % SUMS]);
       }
     }
   }
@@ -193,13 +203,17 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void rmsnorm_reg(
         rout[row * srout + tcol] = vt;
       }
       const float f = to_f32(vt);
-      ss = __builtin_fmaf(f, f, ss);
+      ss[0] = __builtin_fmaf(f, f, ss[0]);
     }
   }
 
   // The weight row is L2-resident (every row reads it); fetch the first group
   // before the reduction so its latency hides behind the cross-lane sums.
+  // The empty asm keeps these loads behind the sums: the compiler otherwise
+  // puts them ahead, and the wait for the row then covers the weights (fp32
+  // rows of 4096, 594 rows 4.4 -> 5.7 us).
   if constexpr (kPrefetchW && !EW) {
+    if constexpr (!RES) asm volatile("" : "+v"(ss[0]) : : "memory");
 #pragma unroll
     for (int k = 0; k < G; ++k) {
       const int vi = t + k * TPR;
@@ -207,16 +221,22 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void rmsnorm_reg(
     }
   }
 
-  ss = wave_sum(ss);
-  if constexpr (WPR > 1) {
-    __shared__ float partial[RPB][WPR];
-    if (lane == 0) partial[row_in_block][wave_in_row] = ss;
-    __syncthreads();
-    ss = 0.f;
 #pragma unroll
-    for (int j = 0; j < WPR; ++j) ss += partial[row_in_block][j];
+  for (int i = 0; i < SUMS; ++i) ss[i] = wave_sum(ss[i]);
+  float total = ss[0];
+  static_assert(SUMS == 1 || WPR > 1, "separate sums meet in LDS");
+  if constexpr (WPR > 1) {
+    __shared__ float partial[RPB][SUMS * WPR];
+    if (lane == 0) {
+#pragma unroll
+      for (int i = 0; i < SUMS; ++i) partial[row_in_block][i * WPR + wave_in_row] = ss[i];
+    }
+    __syncthreads();
+    total = 0.f;
+#pragma unroll
+    for (int j = 0; j < SUMS * WPR; ++j) total += partial[row_in_block][j];
   }
-  const float rstd = rsqrtf(ss * inv_h + eps);
+  const float rstd = rsqrtf(total * inv_h + eps);
 
 #pragma unroll
   for (int g0 = 0; g0 < VPT; g0 += G) {
@@ -273,6 +293,9 @@ __global__ __launch_bounds__(kShortBlock) void rmsnorm_short(
   const int64_t first = row0 + static_cast<int64_t>(blockIdx.x) * (R * U) + threadIdx.x / L;
   const bool has_packet = j < nvec;
   const bool has_tail = j < tail;  // the launcher gives L >= tail lanes
+  // The arguments in one scalar round trip (see rmsnorm_reg).
+  asm volatile("" : : "s"(x), "s"(w), "s"(sx), "s"(y), "s"(sy));
+  if constexpr (RES) asm volatile("" : : "s"(res), "s"(sr), "s"(rout), "s"(srout));
   P v[U];
   [[maybe_unused]] P rv[U];
   T vt[U];
@@ -644,6 +667,7 @@ constexpr int64_t kFewRows = 256;
 
 struct RegShape {
   int wpr, vpt;
+  bool resident = false;  // picked by kResidentLimits
 };
 // Instantiated (waves per row, packets per lane) shapes, smallest first.
 constexpr RegShape kRegShapes[] = {{1, 1}, {1, 2},  {1, 4},  {1, 8},  {2, 1},  {2, 2},  {2, 4},
@@ -654,28 +678,82 @@ constexpr RegShape kRegShapes[] = {{1, 1}, {1, 2},  {1, 4},  {1, 8},  {2, 1},  {
 constexpr int kMaxRegPackets = 16 * 64 * 8;
 
 
-// Default shape (waves per row, packets per lane). Medians of three cold runs
-// per shape on MI355X, 16384 rows, fp16 and bf16: plain rows are fastest
-// with two packets per lane over 4-16 wavefronts; residual rows, which load
-// two tensors per packet, with one packet per lane over 8-16 wavefronts.
-// Rows of at most kShortPackets take rmsnorm_short before this, unless a
-// shape is forced.
-RegShape pick_shape(int64_t nvec, bool residual, int64_t rows) {
-  // One packet per lane and more wavefronts per row for the residual variant,
-  // and for plain rows when a launch has too few rows to give every CU a
-  // workgroup (decode): then each row's latency is the launch's. Graph-replayed
-  // on MI355X, plain rows of 4096 half elements take 1.89 us as (8, 1) against
-  // 2.13 us as (4, 2) at 1 row (2.04 against 2.28 at 32 rows); at 16384 rows
-  // (4, 2) is the faster.
-  const bool one_packet = residual || rows <= kFewRows;
-  RegShape s{16, 8};
-  if (nvec <= 64) s = {1, 1};
-  else if (nvec <= 128) s = {1, 2};
-  else if (nvec <= 256) s = {2, 2};
-  else if (nvec <= 512) s = one_packet ? RegShape{8, 1} : RegShape{4, 2};
-  else if (nvec <= 1024) s = one_packet ? RegShape{16, 1} : RegShape{8, 2};
-  else if (nvec <= 2048) s = {16, 2};
-  else if (nvec <= 4096) s = {16, 4};
+// Shape of a launch of kFewRows to some thousand rows: the one whose wavefronts
+// are resident all at once, so that every row's loads go out at the start and
+// no second round of workgroups waits for the first (a CU holds 32 wavefronts,
+// 24 at eight packets per lane: 8192 and 6144 on the chip). Fewer packets per
+// lane spread a row's latency over more lanes, so the smallest packet count
+// that fits is taken; one packet per lane only while the chip is not much more
+// than half full (a row costs a barrier over all its wavefronts), and never 16
+// wavefronts of more (plain rows of 10240-16384, 279-500 rows: 10-25% behind 8
+// of four). {0, 0} when none fits. Limits from a sweep of every shape over 13 widths x 11 row counts
+// (bf16, cold, MI355X), against the many-row shapes: 5% faster on average for
+// residual and 4% for plain rows. E.g. residual 512 x 4096 5.6 -> 4.5 us, 2048
+// x 4096 14.2 -> 12.0, 4096 x 4096 26.6 -> 22.7, 1024 x 8192 14.1 -> 11.9, 1536
+// x 5120 12.8 -> 11.8; plain 4096 x 3072 11.0 -> 9.1, 4096 x 8192 28.2 -> 24.2,
+// 1024 x 16384 14.6 -> 12.1.
+struct ResidentLimit {
+  int vpt;
+  int64_t plain_waves, residual_waves;
+};
+constexpr ResidentLimit kResidentLimits[] = {{1, 5120, 5632}, {2, 8192, 4096}, {4, 6144, 8192}, {8, 6144, 0}};
+
+// Sums per lane with which a resident shape adds in the order of the streaming
+// shape of the same residual rows: 8 x 1 up to 512 packets, 16 x 1 up to 1024,
+// 16 x 2 up to 2048. Narrower rows keep one sum.
+template <int WPR, int VPT>
+constexpr int kResidentSums = VPT > 4          ? 1
+                              : WPR * VPT == 8 ? 8 / WPR
+                              : WPR * VPT == 16 || WPR * VPT == 32 ? 16 / WPR
+                                                                   : 1;
+
+RegShape pick_resident_shape(int64_t nvec, bool residual, int64_t rows) {
+  for (const ResidentLimit& l : kResidentLimits) {
+    int wpr = 1;
+    while (int64_t(wpr) * kWave * l.vpt < nvec) wpr *= 2;
+    // One packet per lane of residual rows: the wavefronts that hold a packet.
+    const int64_t waves = residual && l.vpt == 1 ? ceil_div(nvec, kWave) : wpr;
+    if (wpr <= (l.vpt == 1 ? 16 : 8) && rows * waves <= (residual ? l.residual_waves : l.plain_waves))
+      return {wpr, l.vpt, true};
+  }
+  return {0, 0};
+}
+
+// Shape of larger launches. Medians of three cold runs per shape on MI355X,
+// 16384 rows, fp16 and bf16: plain rows are fastest with two packets per lane
+// over 4-16 wavefronts; residual rows, which load two tensors per packet, with
+// one packet per lane over 8-16 wavefronts.
+RegShape pick_streaming_shape(int64_t nvec, bool residual) {
+  if (nvec <= 64) return {1, 1};
+  if (nvec <= 128) return {1, 2};
+  if (nvec <= 256) return {2, 2};
+  if (nvec <= 512) return residual ? RegShape{8, 1} : RegShape{4, 2};
+  if (nvec <= 1024) return residual ? RegShape{16, 1} : RegShape{8, 2};
+  if (nvec <= 2048) return {16, 2};
+  return nvec <= 4096 ? RegShape{16, 4} : RegShape{16, 8};
+}
+
+// Shape of launches of at most kFewRows (decode): one packet per lane, a row
+// to a workgroup, since one row's latency is the launch's. Graph-replayed on
+// MI355X, plain rows of 4096 half elements take 1.89 us as (8, 1) against 2.13
+// us as (4, 2) at 1 row (2.04 against 2.28 at 32 rows); residual rows of 1024 /
+// 2048, 32 rows, 2.22 / 2.58 us as (4, 1) against 2.49 / 2.92 us as (1, 2) /
+// (2, 2), plain 256 rows 2.32 / 2.53 against 2.59 / 2.84 us.
+RegShape pick_few_rows_shape(int64_t nvec) {
+  if (nvec <= 256) return {4, 1};
+  if (nvec <= 512) return {8, 1};
+  if (nvec <= 1024) return {16, 1};
+  return pick_streaming_shape(nvec, false);
+}
+
+// Default shape (waves per row, packets per lane), or the forced one. Rows of
+// at most kShortPackets take rmsnorm_short before this, unless a shape is
+// forced. `resident`: whether a shape of kResidentLimits may be taken.
+RegShape pick_shape(int64_t nvec, bool residual, int64_t rows, bool resident) {
+  RegShape s{0, 0};
+  if (rows <= kFewRows) s = pick_few_rows_shape(nvec);
+  else if (resident) s = pick_resident_shape(nvec, residual, rows);
+  if (s.wpr == 0) s = pick_streaming_shape(nvec, residual);
   const int want_wpr = g_rms_tuning.waves_per_row, want_vpt = g_rms_tuning.vecs_per_thread;
   if (want_wpr > 0 || want_vpt > 0) {
     RegShape want{want_wpr > 0 ? want_wpr : s.wpr, want_vpt > 0 ? want_vpt : s.vpt};
@@ -718,7 +796,8 @@ int64_t max_blocks_per_launch(int threads_per_block) {
   return forced > 0 ? std::min(cap, forced) : cap;
 }
 
-template <typename T, typename W, int WPR, int VPT, bool RES, bool EW, bool TAIL, bool SPLIT = false, bool WT = false>
+template <typename T, typename W, int WPR, int VPT, bool RES, bool EW, bool TAIL, int SUMS = 1, bool SPLIT = false,
+          bool WT = false>
 hipError_t run_reg_launch(const RmsArgs& a, hipStream_t stream) {
   constexpr int RPB = WPR >= 4 ? 1 : 4 / WPR;
   const dim3 block(kWave * WPR * RPB);
@@ -748,7 +827,7 @@ hipError_t run_reg_launch(const RmsArgs& a, hipStream_t stream) {
     const int order = g_rms_tuning.row_order, chunk = g_rms_tuning.xcd_chunk;
     if (order == 1) xcd_chunk = 1;
     if (order == 2) xcd_chunk = chunk > 0 ? unsigned(chunk) : unsigned(grid.x / 8);
-    AKO_LAUNCH((rmsnorm_reg<T, W, WPR, VPT, RPB, RES, EW, TAIL, SPLIT, WT>),
+    AKO_LAUNCH((rmsnorm_reg<T, W, WPR, VPT, RPB, RES, EW, TAIL, SUMS, SPLIT, WT>),
                grid, block, lds, stream, static_cast<const T*>(a.x), static_cast<const T*>(a.r),
                static_cast<const W*>(a.w), static_cast<T*>(a.y), static_cast<T*>(a.rout),
                b0 * RPB, a.rows, static_cast<int>(a.hidden), a.sx, a.sr, a.sy, a.srout,
@@ -772,7 +851,7 @@ hipError_t run_reg_launch(const RmsArgs& a, hipStream_t stream) {
 constexpr int64_t kEarlyWeightRowBytes = 8 * 1024;
 
 template <typename T, typename W, int WPR, int VPT, bool RES>
-hipError_t run_reg(const RmsArgs& a, hipStream_t stream) {
+hipError_t run_reg(const RmsArgs& a, bool resident, hipStream_t stream) {
   const bool tail = a.hidden % (16 / static_cast<int>(sizeof(T))) != 0;
   if constexpr (VPT <= 2) {
     const int forced = g_rms_tuning.early_weights;
@@ -781,6 +860,12 @@ hipError_t run_reg(const RmsArgs& a, hipStream_t stream) {
                      a.hidden * static_cast<int64_t>(sizeof(T)) <= kEarlyWeightRowBytes);
     if (ew) return tail ? run_reg_launch<T, W, WPR, VPT, RES, true, true>(a, stream)
                         : run_reg_launch<T, W, WPR, VPT, RES, true, false>(a, stream);
+  }
+  // Resident shapes of residual rows add in the order of the streaming shape.
+  constexpr int kSums = kResidentSums<WPR, VPT>;
+  if constexpr (RES && kSums > 1) {
+    if (resident) return tail ? run_reg_launch<T, W, WPR, VPT, RES, false, true, kSums>(a, stream)
+                              : run_reg_launch<T, W, WPR, VPT, RES, false, false, kSums>(a, stream);
   }
   if (tail) return run_reg_launch<T, W, WPR, VPT, RES, false, true>(a, stream);
   // Without write-through stores (key 12 = 1): one packet per load group for
@@ -806,15 +891,15 @@ hipError_t run_reg(const RmsArgs& a, hipStream_t stream) {
     if (a.aligned16 && (wt_forced == 2 || (wt_forced == 0 && kWtByDefault && a.rows > kFewRows))) {
       if constexpr (RES) {
         if (g_rms_tuning.load_groups != 1)
-          return run_reg_launch<T, W, WPR, VPT, RES, false, false, true, true>(a, stream);
+          return run_reg_launch<T, W, WPR, VPT, RES, false, false, 1, true, true>(a, stream);
       }
-      return run_reg_launch<T, W, WPR, VPT, RES, false, false, false, true>(a, stream);
+      return run_reg_launch<T, W, WPR, VPT, RES, false, false, 1, false, true>(a, stream);
     }
   }
   if constexpr (VPT == 2 && WPR == 16 && RES) {
     const int forced = g_rms_tuning.load_groups;
     const bool split = forced == 2 || (forced == 0 && std::is_same_v<T, __bf16> && a.rows > kFewRows);
-    if (split) return run_reg_launch<T, W, WPR, VPT, RES, false, false, true>(a, stream);
+    if (split) return run_reg_launch<T, W, WPR, VPT, RES, false, false, 1, true>(a, stream);
   }
   return run_reg_launch<T, W, WPR, VPT, RES, false, false>(a, stream);
 }
@@ -835,9 +920,9 @@ int device_cus() {
 }
 
 // Widest input row (x, plus the residual) the pipelined kernel takes by
-// default, and the fewest rows per workgroup at which plain rows take it.
+// default, and the fewest rows per workgroup.
 constexpr int64_t kPipeMaxRowBytes = 16 * 1024;
-constexpr int64_t kPipeMinRowsPerBlock = 16;
+constexpr int64_t kPipeMinRowsPerBlock = 20;
 
 // Shapes with a pipelined instantiation (the defaults of launches of many
 // rows up to 65536 half-precision elements, and their neighbours).
@@ -889,7 +974,7 @@ hipError_t run_pipe_shape(const RegShape& s, const RmsArgs& a, hipStream_t strea
 template <typename T, typename W, bool RES>
 hipError_t run_reg_shape(const RegShape& s, const RmsArgs& a, hipStream_t stream) {
 #define AKO_RMS_SHAPE(WPR, VPT) \
-  if (s.wpr == WPR && s.vpt == VPT) return run_reg<T, W, WPR, VPT, RES>(a, stream);
+  if (s.wpr == WPR && s.vpt == VPT) return run_reg<T, W, WPR, VPT, RES>(a, s.resident, stream);
   AKO_RMS_SHAPE(1, 1)
   AKO_RMS_SHAPE(1, 2)
   AKO_RMS_SHAPE(1, 4)
@@ -995,27 +1080,28 @@ hipError_t run_typed(const RmsArgs& a, hipStream_t stream) {
     return a.residual ? run_short<T, W, true>(a, stream) : run_short<T, W, false>(a, stream);
   const bool reg = g_rms_tuning.force_stream == 0 && nvec <= kMaxRegPackets;
   if (!reg) return a.residual ? run_stream<T, W, true>(a, stream) : run_stream<T, W, false>(a, stream);
-  RegShape s = pick_shape(nvec, a.residual, a.rows);
   // The pipelined kernel takes full rows only (no packet past the row's end)
   // and launches of many rows. By default it runs rows of 512 or 1024
   // packets whose inputs (x, and the residual) total at most 16 KiB, as one
-  // packet per lane per tensor over nvec / 64 wavefronts. Medians of five
-  // cold back-to-back runs on MI355X, 16384 rows, against rmsnorm_reg's
-  // default: plain rows of 4096 half elements 5947 -> 6568 GB/s, residual
-  // rows of 4096 6143 -> 6978, plain rows of 8192 6340 -> 7001, fp32 rows of
-  // 2048 and 4096 +10-15% alike. Rows of 32 KiB of input (residual 8192,
-  // plain and residual 16384), and two packets per lane at any width, were
-  // 3-18% slower pipelined. Plain rows need 16 rows per workgroup: with 2-4
-  // (512 or 2048 rows) they ran 7-15% slower than rmsnorm_reg, while
-  // residual rows were as fast or faster from 300 rows up.
+  // packet per lane per tensor over nvec / 64 wavefronts, once a launch is too
+  // large to be resident at once. Its lead depends on the outputs: 16384
+  // residual rows of 4096 take 76-78 us written over the buffers of the call
+  // before, whose lines the 256 MB MALL still holds, but 98-105 us into buffers
+  // not touched lately, against 86-87 us for rmsnorm_reg either way (plain 4096
+  // 41 and 53 against 44 us, plain 8192 77 and 97 against 84 us). Below 20
+  // rows per workgroup it is level at best: residual 4096 x 4096 23.4 and 26.3
+  // against 22.7 us, plain 4096 x 8192 23.4 and 28.3 against 23.7 us. Rows of
+  // 32 KiB of input (residual 8192, plain and residual 16384), and two packets
+  // per lane at any width, were 3-18% slower pipelined.
   const bool rows_ok = a.rows > kFewRows && a.rows < (int64_t(1) << 31) && nvec * E == a.hidden;
+  RegShape s = pick_shape(nvec, a.residual, a.rows, !(g_rms_tuning.pipeline == 2 && a.residual));
   bool pipe = false;
   if (g_rms_tuning.pipeline == 2) {
     pipe = rows_ok && int64_t(s.wpr) * kWave * s.vpt == nvec && pipe_shape(s);
   } else if (g_rms_tuning.pipeline == 0 && !forced_shape && rows_ok && (nvec == 512 || nvec == 1024) &&
              a.hidden * static_cast<int64_t>(sizeof(T)) * (a.residual ? 2 : 1) <= kPipeMaxRowBytes) {
     const RegShape one{static_cast<int>(nvec / kWave), 1};
-    if (a.residual || a.rows >= kPipeMinRowsPerBlock * pipe_blocks(one.wpr, false, a.rows)) {
+    if (a.rows >= kPipeMinRowsPerBlock * pipe_blocks(one.wpr, a.residual, a.rows)) {
       s = one;
       pipe = true;
     }
