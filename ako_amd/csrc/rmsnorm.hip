@@ -583,7 +583,12 @@ __global__ __launch_bounds__(kStreamBlock) void rmsnorm_shard_partial(
       const P q = load_pack<T, E, true>(res + row * sr + vi * E);
 #pragma unroll
       for (int e = 0; e < E; ++e) p.e[e] = from_f32<T>(to_f32(p.e[e]) + to_f32(q.e[e]));
-      store_pack<T, E, true>(rout + row * srout + vi * E, p);
+      // No non-temporal hint: the apply half reads s again as soon as the sums
+      // are in, and finds in the MALL what this half wrote last. Both halves,
+      // MI355X, bf16, residual: 16384 rows of 1024 / 2048 / 4096 / 8192 33.6 /
+      // 57.0 / 110.6 / 232.7 -> 31.7 / 55.0 / 101.7 / 206.1 us, 2048 rows of
+      // 2048 11.8 -> 11.0 us (this half alone 31.8 -> 32.4 us at 2048).
+      store_pack<T, E>(rout + row * srout + vi * E, p);
     }
     ss = sumsq_add(p, ss);
   }
@@ -611,12 +616,12 @@ __global__ __launch_bounds__(kStreamBlock) void rmsnorm_shard_partial(
 template <typename T, typename W, int R>
 __global__ __launch_bounds__(kStreamBlock) void rmsnorm_shard_apply(
     const T* __restrict__ s, const W* __restrict__ w, const float* __restrict__ total,
-    T* __restrict__ y, int64_t row0, int64_t rows, int shard, int64_t ss_, int64_t sy, float inv_h, float eps) {
-  // Each workgroup applies R consecutive rows; a lane holds the same columns of
-  // all R, so the weight packet is read once for R rows.
+    T* __restrict__ y, int64_t row0, int64_t rows, int64_t apart, int shard, int64_t ss_, int64_t sy, float inv_h, float eps) {
+  // Each workgroup applies R rows `apart` rows from each other; a lane holds the
+  // same columns of all R, so the weight packet is read once for R rows.
   constexpr int E = 16 / static_cast<int>(sizeof(T));
   using P = Pack<T, E>;
-  const int64_t first = row0 + static_cast<int64_t>(blockIdx.x) * R;
+  const int64_t first = row0 + blockIdx.x;
   const int tid = threadIdx.x;
   const int nvec = shard / E;
   const auto apply = [&](int64_t row, int vi, const P& p, const float (&wf)[E], float rstd) {
@@ -634,23 +639,23 @@ __global__ __launch_bounds__(kStreamBlock) void rmsnorm_shard_apply(
     P p[R];
 #pragma unroll
     for (int k = 0; k < R; ++k)
-      if (first + k < rows) p[k] = load_pack<T, E, true>(s + (first + k) * ss_ + vi * E);
+      if (first + k * apart < rows) p[k] = load_pack<T, E, true>(s + (first + k * apart) * ss_ + vi * E);
     float wf[E];
     load_f32<W, E>(w + vi * E, wf);
     if (!have_rstd) {
 #pragma unroll
-      for (int k = 0; k < R; ++k) rstd[k] = first + k < rows ? rsqrtf(total[first + k] * inv_h + eps) : 0.f;
+      for (int k = 0; k < R; ++k) rstd[k] = first + k * apart < rows ? rsqrtf(total[first + k * apart] * inv_h + eps) : 0.f;
       have_rstd = true;
     }
 #pragma unroll
     for (int k = 0; k < R; ++k)
-      if (first + k < rows) apply(first + k, vi, p[k], wf, rstd[k]);
+      if (first + k * apart < rows) apply(first + k * apart, vi, p[k], wf, rstd[k]);
   }
   const int tail0 = nvec * E + tid;
   if (tail0 < shard) {
 #pragma unroll
     for (int k = 0; k < R; ++k) {
-      const int64_t row = first + k;
+      const int64_t row = first + k * apart;
       if (row >= rows) break;
       const float rs = rsqrtf(total[row] * inv_h + eps);
       const T* sr = s + row * ss_;
@@ -1135,9 +1140,15 @@ hipError_t run_shard_apply_r(const RmsShardArgs& a, hipStream_t stream) {
   const float inv_h = 1.0f / static_cast<float>(a.hidden);
   for (int64_t r0 = 0; r0 < a.rows; r0 += cap) {
     const int64_t end = std::min(a.rows, r0 + cap);
-    const dim3 grid(static_cast<unsigned>(ceil_div(end - r0, R)));
+    // Rows a multiple of 8 apart: their workgroup runs on the XCD whose
+    // workgroups of the partial half wrote them (workgroup b runs on XCD b % 8),
+    // and finds what is left of them in its L2 (both halves, outputs over those
+    // of the call before, 4096 rows of 2048: 21.2 us with neighbouring rows,
+    // 15.7 us so).
+    const int64_t apart = R == 1 ? end - r0 : ceil_div(ceil_div(end - r0, R), 8) * 8;
+    const dim3 grid(static_cast<unsigned>(std::min(apart, end - r0)));
     AKO_LAUNCH((rmsnorm_shard_apply<T, W, R>), grid, dim3(kStreamBlock), 0, stream,
-               static_cast<const T*>(a.x), static_cast<const W*>(a.w), a.total, static_cast<T*>(a.y), r0, end,
+               static_cast<const T*>(a.x), static_cast<const W*>(a.w), a.total, static_cast<T*>(a.y), r0, end, apart,
                static_cast<int>(a.shard), a.sx, a.sy, inv_h, a.eps);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;

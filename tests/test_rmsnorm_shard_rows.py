@@ -1,0 +1,25 @@
+"""The apply half of the sharded RMSNorm at the row counts where a workgroup
+takes two rows (4096 up), a multiple of 8 rows apart: even, odd and ragged
+halves, each row the same as in a launch of one row per workgroup."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from ako_amd.ops.rmsnorm_tp import rmsnorm_shard_apply_hip, rmsnorm_shard_partial_hip
+
+pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")]
+
+
+@pytest.mark.parametrize("rows", [4095, 4096, 4097, 4103, 4104, 8191])
+@pytest.mark.parametrize("width", [8, 264, 515])
+def test_two_rows_per_workgroup(rows: int, width: int) -> None:
+    gen = torch.Generator(device="cuda").manual_seed(rows + width)
+    x, r = (torch.randn(rows, width, generator=gen, device="cuda").to(torch.bfloat16) for _ in range(2))
+    w = torch.randn(width, generator=gen, device="cuda").to(torch.bfloat16)
+    s, sums = rmsnorm_shard_partial_hip(x, r)
+    assert torch.equal(s, x + r)
+    y = rmsnorm_shard_apply_hip(s, w, sums, 4 * width)
+    parts = [rmsnorm_shard_apply_hip(s[i:i + 1000], w, sums[i:i + 1000], 4 * width) for i in range(0, rows, 1000)]
+    assert torch.equal(y, torch.cat(parts))
