@@ -164,6 +164,12 @@ class KernelSelector:
         call_kwargs: dict[str, Any] | None = None,
     ) -> KernelFn:
         """The callable to run for this call; memoised on cheap hashables."""
+        if forced:  # the same kernel whatever the tensors: no need to look at them
+            fn = self._memo.get((op_name, forced))
+            if fn is None:
+                fn = self.select_entry(op_name, x, *args, forced=forced, extra_key=extra_key).entry.fn
+                self._memo[(op_name, forced)] = fn
+            return fn
         memo_key = (
             op_name,
             forced,
