@@ -14,10 +14,11 @@
 //   residual) written once, all with the non-temporal hint; the weight row
 //   is re-read by every row and stays in L2. The sum of squares is reduced
 //   in fp32 with DPP inside the wavefront and, when WPR > 1, through WPR
-//   floats of LDS. Small rows pack RPB rows into one workgroup. A lane issues every load of a group of packets
-//   before consuming any of them, so its memory latency is paid once per
-//   group instead of once per packet. Wide rows are handed to the 8 XCDs in
-//   runs of consecutive rows (block_order) rather than row by row.
+//   floats of LDS. Small rows pack RPB rows into one workgroup. A lane issues
+//   every load of a group of packets before consuming any of them, so its
+//   memory latency is paid once per group instead of once per packet. Wide rows
+//   are handed to the 8 XCDs in runs of consecutive rows (block_order) rather
+//   than row by row.
 //
 // rmsnorm_pipe - rmsnorm_reg's row layout in a persistent, software-pipelined
 //   grid: each workgroup walks a sequence of rows and issues the next row's
@@ -51,6 +52,7 @@
 
 #include "common.h"
 #include "launch.h"
+#include "rmsnorm_rule.h"
 
 namespace ako {
 
@@ -224,8 +226,10 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void rmsnorm_reg(
 #pragma unroll
   for (int i = 0; i < SUMS; ++i) ss[i] = wave_sum(ss[i]);
   float total = ss[0];
-  static_assert(SUMS == 1 || WPR > 1, "separate sums meet in LDS");
-  if constexpr (WPR > 1) {
+  if constexpr (WPR == 1) {
+#pragma unroll
+    for (int i = 1; i < SUMS; ++i) total += ss[i];
+  } else {
     __shared__ float partial[RPB][SUMS * WPR];
     if (lane == 0) {
 #pragma unroll
@@ -667,107 +671,6 @@ __global__ __launch_bounds__(kStreamBlock) void rmsnorm_shard_apply(
 
 namespace {
 
-// Launches of at most this many rows leave CUs without a workgroup (256 CUs).
-constexpr int64_t kFewRows = 256;
-
-struct RegShape {
-  int wpr, vpt;
-  bool resident = false;  // picked by kResidentLimits
-};
-// Instantiated (waves per row, packets per lane) shapes, smallest first.
-constexpr RegShape kRegShapes[] = {{1, 1}, {1, 2},  {1, 4},  {1, 8},  {2, 1},  {2, 2},  {2, 4},
-                                   {2, 8}, {4, 1},  {4, 2},  {4, 4},  {4, 8},  {8, 1},  {8, 2},
-                                   {8, 4}, {8, 8},  {16, 1}, {16, 2}, {16, 4}, {16, 8}};
-// Widest row held in registers: 16 wavefronts x 64 lanes x 8 packets (65536
-// half-precision elements). Wider rows take the two-pass kernel.
-constexpr int kMaxRegPackets = 16 * 64 * 8;
-
-
-// Shape of a launch of kFewRows to some thousand rows: the one whose wavefronts
-// are resident all at once, so that every row's loads go out at the start and
-// no second round of workgroups waits for the first (a CU holds 32 wavefronts,
-// 24 at eight packets per lane: 8192 and 6144 on the chip). Fewer packets per
-// lane spread a row's latency over more lanes, so the smallest packet count
-// that fits is taken; one packet per lane only while the chip is not much more
-// than half full (a row costs a barrier over all its wavefronts), and never 16
-// wavefronts of more (plain rows of 10240-16384, 279-500 rows: 10-25% behind 8
-// of four). {0, 0} when none fits. Limits from a sweep of every shape over 13 widths x 11 row counts
-// (bf16, cold, MI355X), against the many-row shapes: 5% faster on average for
-// residual and 4% for plain rows. E.g. residual 512 x 4096 5.6 -> 4.5 us, 2048
-// x 4096 14.2 -> 12.0, 4096 x 4096 26.6 -> 22.7, 1024 x 8192 14.1 -> 11.9, 1536
-// x 5120 12.8 -> 11.8; plain 4096 x 3072 11.0 -> 9.1, 4096 x 8192 28.2 -> 24.2,
-// 1024 x 16384 14.6 -> 12.1.
-struct ResidentLimit {
-  int vpt;
-  int64_t plain_waves, residual_waves;
-};
-constexpr ResidentLimit kResidentLimits[] = {{1, 5120, 5632}, {2, 8192, 4096}, {4, 6144, 8192}, {8, 6144, 0}};
-
-// Sums per lane with which a resident shape adds in the order of the streaming
-// shape of the same residual rows: 8 x 1 up to 512 packets, 16 x 1 up to 1024,
-// 16 x 2 up to 2048. Narrower rows keep one sum.
-template <int WPR, int VPT>
-constexpr int kResidentSums = VPT > 4          ? 1
-                              : WPR * VPT == 8 ? 8 / WPR
-                              : WPR * VPT == 16 || WPR * VPT == 32 ? 16 / WPR
-                                                                   : 1;
-
-RegShape pick_resident_shape(int64_t nvec, bool residual, int64_t rows) {
-  for (const ResidentLimit& l : kResidentLimits) {
-    int wpr = 1;
-    while (int64_t(wpr) * kWave * l.vpt < nvec) wpr *= 2;
-    // One packet per lane of residual rows: the wavefronts that hold a packet.
-    const int64_t waves = residual && l.vpt == 1 ? ceil_div(nvec, kWave) : wpr;
-    if (wpr <= (l.vpt == 1 ? 16 : 8) && rows * waves <= (residual ? l.residual_waves : l.plain_waves))
-      return {wpr, l.vpt, true};
-  }
-  return {0, 0};
-}
-
-// Shape of larger launches. Medians of three cold runs per shape on MI355X,
-// 16384 rows, fp16 and bf16: plain rows are fastest with two packets per lane
-// over 4-16 wavefronts; residual rows, which load two tensors per packet, with
-// one packet per lane over 8-16 wavefronts.
-RegShape pick_streaming_shape(int64_t nvec, bool residual) {
-  if (nvec <= 64) return {1, 1};
-  if (nvec <= 128) return {1, 2};
-  if (nvec <= 256) return {2, 2};
-  if (nvec <= 512) return residual ? RegShape{8, 1} : RegShape{4, 2};
-  if (nvec <= 1024) return residual ? RegShape{16, 1} : RegShape{8, 2};
-  if (nvec <= 2048) return {16, 2};
-  return nvec <= 4096 ? RegShape{16, 4} : RegShape{16, 8};
-}
-
-// Shape of launches of at most kFewRows (decode): one packet per lane, a row
-// to a workgroup, since one row's latency is the launch's. Graph-replayed on
-// MI355X, plain rows of 4096 half elements take 1.89 us as (8, 1) against 2.13
-// us as (4, 2) at 1 row (2.04 against 2.28 at 32 rows); residual rows of 1024 /
-// 2048, 32 rows, 2.22 / 2.58 us as (4, 1) against 2.49 / 2.92 us as (1, 2) /
-// (2, 2), plain 256 rows 2.32 / 2.53 against 2.59 / 2.84 us.
-RegShape pick_few_rows_shape(int64_t nvec) {
-  if (nvec <= 256) return {4, 1};
-  if (nvec <= 512) return {8, 1};
-  if (nvec <= 1024) return {16, 1};
-  return pick_streaming_shape(nvec, false);
-}
-
-// Default shape (waves per row, packets per lane), or the forced one. Rows of
-// at most kShortPackets take rmsnorm_short before this, unless a shape is
-// forced. `resident`: whether a shape of kResidentLimits may be taken.
-RegShape pick_shape(int64_t nvec, bool residual, int64_t rows, bool resident) {
-  RegShape s{0, 0};
-  if (rows <= kFewRows) s = pick_few_rows_shape(nvec);
-  else if (resident) s = pick_resident_shape(nvec, residual, rows);
-  if (s.wpr == 0) s = pick_streaming_shape(nvec, residual);
-  const int want_wpr = g_rms_tuning.waves_per_row, want_vpt = g_rms_tuning.vecs_per_thread;
-  if (want_wpr > 0 || want_vpt > 0) {
-    RegShape want{want_wpr > 0 ? want_wpr : s.wpr, want_vpt > 0 ? want_vpt : s.vpt};
-    for (const RegShape& c : kRegShapes)
-      if (c.wpr == want.wpr && c.vpt == want.vpt && int64_t(c.wpr) * 64 * c.vpt >= nvec) return c;
-  }
-  return s;
-}
-
 constexpr unsigned kXcdChunk = 8;
 // Residual rows of 16384 half elements (the one-workgroup-per-CU launches
 // below, write-through stores, one packet per load group) take runs of 16.
@@ -856,8 +759,14 @@ hipError_t run_reg_launch(const RmsArgs& a, hipStream_t stream) {
 constexpr int64_t kEarlyWeightRowBytes = 8 * 1024;
 
 template <typename T, typename W, int WPR, int VPT, bool RES>
-hipError_t run_reg(const RmsArgs& a, bool resident, hipStream_t stream) {
+hipError_t run_reg(const RmsArgs& a, int sums, hipStream_t stream) {
   const bool tail = a.hidden % (16 / static_cast<int>(sizeof(T))) != 0;
+  constexpr int kSums = reg_sums(WPR, VPT, RES);
+  if constexpr (kSums > 1) {
+    if (sums == kSums) return tail ? run_reg_launch<T, W, WPR, VPT, RES, false, true, kSums>(a, stream)
+                                   : run_reg_launch<T, W, WPR, VPT, RES, false, false, kSums>(a, stream);
+  }
+  if (sums != 1) return hipErrorInvalidValue;
   if constexpr (VPT <= 2) {
     const int forced = g_rms_tuning.early_weights;
     const bool ew = forced == 2 ||
@@ -865,12 +774,6 @@ hipError_t run_reg(const RmsArgs& a, bool resident, hipStream_t stream) {
                      a.hidden * static_cast<int64_t>(sizeof(T)) <= kEarlyWeightRowBytes);
     if (ew) return tail ? run_reg_launch<T, W, WPR, VPT, RES, true, true>(a, stream)
                         : run_reg_launch<T, W, WPR, VPT, RES, true, false>(a, stream);
-  }
-  // Resident shapes of residual rows add in the order of the streaming shape.
-  constexpr int kSums = kResidentSums<WPR, VPT>;
-  if constexpr (RES && kSums > 1) {
-    if (resident) return tail ? run_reg_launch<T, W, WPR, VPT, RES, false, true, kSums>(a, stream)
-                              : run_reg_launch<T, W, WPR, VPT, RES, false, false, kSums>(a, stream);
   }
   if (tail) return run_reg_launch<T, W, WPR, VPT, RES, false, true>(a, stream);
   // Without write-through stores (key 12 = 1): one packet per load group for
@@ -924,36 +827,9 @@ int device_cus() {
   return n;
 }
 
-// Widest input row (x, plus the residual) the pipelined kernel takes by
-// default, and the fewest rows per workgroup.
-constexpr int64_t kPipeMaxRowBytes = 16 * 1024;
-constexpr int64_t kPipeMinRowsPerBlock = 20;
-
-// Shapes with a pipelined instantiation (the defaults of launches of many
-// rows up to 65536 half-precision elements, and their neighbours).
-constexpr RegShape kPipeShapes[] = {{4, 2}, {8, 1}, {8, 2}, {16, 1}, {16, 2}, {16, 4}};
-
-bool pipe_shape(const RegShape& s) {
-  for (const RegShape& c : kPipeShapes)
-    if (c.wpr == s.wpr && c.vpt == s.vpt) return true;
-  return false;
-}
-
-// Workgroups of a pipelined launch (a multiple of 8). Workgroups per CU: 16
-// wavefronts per CU for plain rows, 8 for residual rows (two tensors in
-// flight per row). Measured at 16384 rows of 4096 half elements: plain 6598
-// GB/s with 16 wavefronts per CU against 6029 with 8; residual 6976 with 8
-// against 6826 with 16.
-int64_t pipe_blocks(int wpr, bool residual, int64_t rows) {
-  const int forced = g_rms_tuning.pipe_blocks_per_cu;
-  const int64_t per_cu = forced > 0 ? forced : std::max(1, (residual ? 8 : 16) / wpr);
-  const int64_t blocks = std::min<int64_t>(rows, per_cu * device_cus());
-  return std::max<int64_t>(8, blocks / 8 * 8);
-}
-
 template <typename T, typename W, int WPR, int VPT, bool RES>
 hipError_t run_pipe(const RmsArgs& a, hipStream_t stream) {
-  const int64_t blocks = pipe_blocks(WPR, RES, a.rows);
+  const int64_t blocks = pipe_blocks(WPR, RES, a.rows, device_cus(), g_rms_tuning.pipe_blocks_per_cu);
   const int xcd_runs = g_rms_tuning.row_order == 1 ? 0 : 1;
   AKO_LAUNCH((rmsnorm_pipe<T, W, WPR, VPT, RES>), dim3(static_cast<unsigned>(blocks)), dim3(kWave * WPR),
              0, stream, static_cast<const T*>(a.x), static_cast<const T*>(a.r),
@@ -977,9 +853,9 @@ hipError_t run_pipe_shape(const RegShape& s, const RmsArgs& a, hipStream_t strea
 }
 
 template <typename T, typename W, bool RES>
-hipError_t run_reg_shape(const RegShape& s, const RmsArgs& a, hipStream_t stream) {
+hipError_t run_reg_shape(const RegShape& s, int sums, const RmsArgs& a, hipStream_t stream) {
 #define AKO_RMS_SHAPE(WPR, VPT) \
-  if (s.wpr == WPR && s.vpt == VPT) return run_reg<T, W, WPR, VPT, RES>(a, s.resident, stream);
+  if (s.wpr == WPR && s.vpt == VPT) return run_reg<T, W, WPR, VPT, RES>(a, sums, stream);
   AKO_RMS_SHAPE(1, 1)
   AKO_RMS_SHAPE(1, 2)
   AKO_RMS_SHAPE(1, 4)
@@ -1023,9 +899,6 @@ hipError_t run_stream(const RmsArgs& a, hipStream_t stream) {
   }
   return hipSuccess;
 }
-
-// Widest row (in packets) of rmsnorm_short.
-constexpr int kShortPackets = 64;
 
 template <typename T, typename W, int L, int U, bool RES>
 hipError_t run_short_groups(const RmsArgs& a, hipStream_t stream) {
@@ -1076,44 +949,27 @@ hipError_t run_short(const RmsArgs& a, hipStream_t stream) {
   return run_short_lanes<T, W, 64, RES>(a, stream);
 }
 
+template <typename T, typename W, bool RES>
+hipError_t run_route(const RmsArgs& a, hipStream_t stream) {
+  constexpr int E = 16 / sizeof(T);
+  const RmsTuning& k = g_rms_tuning;
+  const NormRoute route = norm_route(
+      {a.hidden / E, a.hidden % E == 0, a.hidden * static_cast<int64_t>(sizeof(T)), a.rows, RES,
+       a.rows > kFewRows ? device_cus() : 0},  // few rows: not looked at
+      {k.waves_per_row, k.vecs_per_thread, k.force_stream, k.early_weights, k.pipeline, k.pipe_blocks_per_cu,
+       k.load_groups, k.write_through});
+  switch (route.kernel) {
+    case NormKernel::kShort: return run_short<T, W, RES>(a, stream);
+    case NormKernel::kReg: return run_reg_shape<T, W, RES>(route.shape, route.sums, a, stream);
+    case NormKernel::kPipe: return run_pipe_shape<T, W, RES>(route.shape, a, stream);
+    case NormKernel::kStream: return run_stream<T, W, RES>(a, stream);
+  }
+  return hipErrorInvalidValue;
+}
+
 template <typename T, typename W>
 hipError_t run_typed(const RmsArgs& a, hipStream_t stream) {
-  constexpr int E = 16 / sizeof(T);
-  const int64_t nvec = a.hidden / E;
-  const bool forced_shape = g_rms_tuning.waves_per_row > 0 || g_rms_tuning.vecs_per_thread > 0;
-  if (nvec <= kShortPackets && !forced_shape && g_rms_tuning.force_stream == 0)
-    return a.residual ? run_short<T, W, true>(a, stream) : run_short<T, W, false>(a, stream);
-  const bool reg = g_rms_tuning.force_stream == 0 && nvec <= kMaxRegPackets;
-  if (!reg) return a.residual ? run_stream<T, W, true>(a, stream) : run_stream<T, W, false>(a, stream);
-  // The pipelined kernel takes full rows only (no packet past the row's end)
-  // and launches of many rows. By default it runs rows of 512 or 1024
-  // packets whose inputs (x, and the residual) total at most 16 KiB, as one
-  // packet per lane per tensor over nvec / 64 wavefronts, once a launch is too
-  // large to be resident at once. Its lead depends on the outputs: 16384
-  // residual rows of 4096 take 76-78 us written over the buffers of the call
-  // before, whose lines the 256 MB MALL still holds, but 98-105 us into buffers
-  // not touched lately, against 86-87 us for rmsnorm_reg either way (plain 4096
-  // 41 and 53 against 44 us, plain 8192 77 and 97 against 84 us). Below 20
-  // rows per workgroup it is level at best: residual 4096 x 4096 23.4 and 26.3
-  // against 22.7 us, plain 4096 x 8192 23.4 and 28.3 against 23.7 us. Rows of
-  // 32 KiB of input (residual 8192, plain and residual 16384), and two packets
-  // per lane at any width, were 3-18% slower pipelined.
-  const bool rows_ok = a.rows > kFewRows && a.rows < (int64_t(1) << 31) && nvec * E == a.hidden;
-  RegShape s = pick_shape(nvec, a.residual, a.rows, !(g_rms_tuning.pipeline == 2 && a.residual));
-  bool pipe = false;
-  if (g_rms_tuning.pipeline == 2) {
-    pipe = rows_ok && int64_t(s.wpr) * kWave * s.vpt == nvec && pipe_shape(s);
-  } else if (g_rms_tuning.pipeline == 0 && !forced_shape && rows_ok && (nvec == 512 || nvec == 1024) &&
-             a.hidden * static_cast<int64_t>(sizeof(T)) * (a.residual ? 2 : 1) <= kPipeMaxRowBytes) {
-    const RegShape one{static_cast<int>(nvec / kWave), 1};
-    if (a.rows >= kPipeMinRowsPerBlock * pipe_blocks(one.wpr, a.residual, a.rows)) {
-      s = one;
-      pipe = true;
-    }
-  }
-  if (pipe) return a.residual ? run_pipe_shape<T, W, true>(s, a, stream) : run_pipe_shape<T, W, false>(s, a, stream);
-  return a.residual ? run_reg_shape<T, W, true>(s, a, stream)
-                    : run_reg_shape<T, W, false>(s, a, stream);
+  return a.residual ? run_route<T, W, true>(a, stream) : run_route<T, W, false>(a, stream);
 }
 
 }  // namespace

@@ -1,0 +1,213 @@
+// Which RMSNorm kernel a launch takes, in which shape, and in which order it
+// adds a row's squares. Plain C++ (no HIP), so that a CPU test can walk the
+// whole rule.
+//
+// The order is settled first, from the row's width and the kind of launch,
+// and the shape only among those that can add in it: a faster shape never
+// changes a result. A residual row adds in one order at every launch size, and
+// so does a plain row of at most 256 packets; a plain row of 257-1024 packets
+// has one order in launches of at most kFewRows rows and in those of the
+// pipelined kernel's size, and another one between.
+#pragma once
+
+#include <stdint.h>
+
+namespace ako {
+
+// Launches of at most this many rows leave CUs without a workgroup (256 CUs).
+constexpr int64_t kFewRows = 256;
+
+// Widest row (in packets) of rmsnorm_short.
+constexpr int64_t kShortPackets = 64;
+
+// Widest row held in registers: 16 wavefronts x 64 lanes x 8 packets (65536
+// half-precision elements). Wider rows take the two-pass kernel.
+constexpr int64_t kMaxRegPackets = 16 * 64 * 8;
+
+// Wavefronts per row and packets per lane.
+struct RegShape {
+  int wpr, vpt;
+};
+// Instantiated shapes, smallest first.
+constexpr RegShape kRegShapes[] = {{1, 1}, {1, 2},  {1, 4},  {1, 8},  {2, 1},  {2, 2},  {2, 4},
+                                   {2, 8}, {4, 1},  {4, 2},  {4, 4},  {4, 8},  {8, 1},  {8, 2},
+                                   {8, 4}, {8, 8},  {16, 1}, {16, 2}, {16, 4}, {16, 8}};
+
+// Separate sums per lane of a register shape that adds in the order of a wider
+// one (see rmsnorm_reg); every shape has this one variant beside the one with
+// a single sum. The order of `total` = wavefronts x packets: plain rows add as
+// 2 x 2, 4 x 2, 8 x 2, 16 x 2 or 16 x 4, residual rows as 2 x 2, 8 x 1, 16 x 1
+// or 16 x 2. Plain 4 x 2 and 8 x 2 themselves stand in for 8 x 1 and 16 x 1.
+constexpr int reg_sums(int wpr, int vpt, bool residual) {
+  const int total = wpr * vpt;
+  if (residual && vpt > 4) return 1;  // not among the resident shapes of residual rows
+  int order = 0;                      // wavefronts of the order
+  if (total == 4) order = 2;
+  if (total == 8) order = residual || vpt == 2 ? 8 : 4;
+  if (total == 16) order = residual || vpt == 2 ? 16 : 8;
+  if (total == 32) order = 16;
+  if (total == 64) order = 16;
+  return order > wpr ? order / wpr : 1;
+}
+
+// Wavefronts and packets of the order in which a launch adds. `one_packet`:
+// plain rows of 257-1024 packets take one packet per lane, as residual rows do.
+//
+// These are also the shapes of large launches (with the plain rows that a
+// large launch holds at two packets per lane). Medians of three cold runs per
+// shape on MI355X, 16384 rows, fp16 and bf16: plain rows are fastest with two
+// packets per lane over 4-16 wavefronts; residual rows, which load two tensors
+// per packet, with one packet per lane over 8-16 wavefronts. Launches of at
+// most kFewRows (decode) take one packet per lane, a row to a workgroup, since
+// one row's latency is the launch's: graph-replayed on MI355X, plain rows of
+// 4096 half elements take 1.89 us as (8, 1) against 2.13 us as (4, 2) at 1 row
+// (2.04 against 2.28 at 32 rows). Rows of 65-256 packets would gain by it too
+// (bf16, cold, (4, 1) against these shapes: 32 rows of 2048, plain 2.52 and 2.89
+// us, residual 2.85 and 3.33; 300 rows 2.83 and 3.11, 3.25 and 3.79), as would
+// plain rows of 257-512 packets above kFewRows ((8, 1) against (4, 2): 300 x 4096
+// 3.27 and 3.43 us), but not in the order of their larger launches.
+inline RegShape sum_order(int64_t nvec, bool one_packet) {
+  if (nvec <= 64) return {1, 1};
+  if (nvec <= 128) return {1, 2};
+  if (nvec <= 256) return {2, 2};
+  if (nvec <= 512) return one_packet ? RegShape{8, 1} : RegShape{4, 2};
+  if (nvec <= 1024) return one_packet ? RegShape{16, 1} : RegShape{8, 2};
+  if (nvec <= 2048) return {16, 2};
+  return nvec <= 4096 ? RegShape{16, 4} : RegShape{16, 8};
+}
+
+// Shape of a launch of kFewRows to some thousand rows: the one whose wavefronts
+// are resident all at once, so that every row's loads go out at the start and
+// no second round of workgroups waits for the first (a CU holds 32 wavefronts,
+// 24 at eight packets per lane: 8192 and 6144 on the chip). Fewer packets per
+// lane spread a row's latency over more lanes, so the smallest packet count
+// that fits and adds in the row's order is taken, and never 16 wavefronts of
+// more than one packet (plain rows of 10240-16384, 279-500 rows: 10-25% behind
+// 8 of four). Limits from a sweep of every shape over 13 widths x 11 row
+// counts (bf16, cold, MI355X). E.g. against the many-row shapes: residual 512 x
+// 4096 5.6 -> 4.5 us, 2048 x 4096 14.2 -> 12.0, 4096 x 4096 26.6 -> 22.7, 1024 x
+// 8192 14.1 -> 11.9, 1536 x 5120 12.8 -> 11.8; plain 4096 x 3072 11.0 -> 9.1,
+// 1024 x 16384 14.6 -> 12.1.
+struct ResidentLimit {
+  int vpt;
+  int64_t plain_waves, residual_waves;
+};
+constexpr ResidentLimit kResidentLimits[] = {{1, 5120, 5632}, {2, 8192, 4096}, {4, 6144, 8192}, {8, 6144, 0}};
+
+// A shape of kResidentLimits that adds in `order`, or {0, 0}. Such a shape
+// holds as many packets over fewer wavefronts, with more sums per lane.
+inline RegShape resident_shape(RegShape order, int64_t nvec, bool residual, int64_t rows) {
+  const int total = order.wpr * order.vpt;
+  for (const ResidentLimit& l : kResidentLimits) {
+    const int wpr = total / l.vpt;
+    if (wpr < 1 || wpr > order.wpr || wpr > (l.vpt == 1 ? 16 : 8)) continue;
+    // One packet per lane of residual rows: the wavefronts that hold a packet.
+    const int64_t waves = residual && l.vpt == 1 ? (nvec + 63) / 64 : wpr;
+    if (rows * waves <= (residual ? l.residual_waves : l.plain_waves)) return {wpr, l.vpt};
+  }
+  return {0, 0};
+}
+
+// Widest input row (x, plus the residual) the pipelined kernel takes by
+// default, the fewest rows per workgroup, and the fewest at which plain rows
+// add in its order.
+constexpr int64_t kPipeMaxRowBytes = 16 * 1024;
+constexpr int64_t kPipeMinRowsPerBlock = 20;
+constexpr int64_t kPipeOrderRowsPerBlock = 16;
+
+// Shapes with a pipelined instantiation (those of launches of many rows up to
+// 65536 half-precision elements, and their neighbours).
+constexpr RegShape kPipeShapes[] = {{4, 2}, {8, 1}, {8, 2}, {16, 1}, {16, 2}, {16, 4}};
+
+inline bool pipe_shape(const RegShape& s) {
+  for (const RegShape& c : kPipeShapes)
+    if (c.wpr == s.wpr && c.vpt == s.vpt) return true;
+  return false;
+}
+
+// What the rule looks at, of the launch and of the tuning keys (see RmsTuning).
+struct NormCall {
+  int64_t nvec;       // whole packets per row
+  bool full;          // no partial packet
+  int64_t row_bytes;  // of one tensor
+  int64_t rows;
+  bool residual;
+  int cus;
+};
+struct NormKeys {
+  int waves_per_row, vecs_per_thread, force_stream, early_weights, pipeline, pipe_blocks_per_cu, load_groups,
+      write_through;
+};
+
+// Workgroups of a pipelined launch (a multiple of 8). Workgroups per CU: 16
+// wavefronts per CU for plain rows, 8 for residual rows (two tensors in
+// flight per row). Measured at 16384 rows of 4096 half elements: plain 6598
+// GB/s with 16 wavefronts per CU against 6029 with 8; residual 6976 with 8
+// against 6826 with 16.
+inline int64_t pipe_blocks(int wpr, bool residual, int64_t rows, int cus, int forced_per_cu) {
+  const int waves = residual ? 8 : 16;
+  const int64_t per_cu = forced_per_cu > 0 ? forced_per_cu : wpr < waves ? waves / wpr : 1;
+  const int64_t blocks = per_cu * cus < rows ? per_cu * cus : rows;
+  return blocks >= 16 ? blocks / 8 * 8 : 8;
+}
+
+enum class NormKernel { kShort, kReg, kPipe, kStream };
+struct NormRoute {
+  NormKernel kernel;
+  RegShape shape;  // kReg and kPipe
+  int sums;        // kReg: sums per lane
+};
+
+// Rows of at most kShortPackets take rmsnorm_short unless a shape is forced.
+//
+// The pipelined kernel takes full rows only (no packet past the row's end)
+// and launches of many rows. By default it runs rows of 512 or 1024
+// packets whose inputs (x, and the residual) total at most 16 KiB, as one
+// packet per lane per tensor over nvec / 64 wavefronts, once a launch is too
+// large to be resident at once. Its lead depends on the outputs: 16384
+// residual rows of 4096 take 76-78 us written over the buffers of the call
+// before, whose lines the 256 MB MALL still holds, but 98-105 us into buffers
+// not touched lately, against 86-87 us for rmsnorm_reg either way (plain 4096
+// 41 and 53 against 44 us, plain 8192 77 and 97 against 84 us). Below 20
+// rows per workgroup it is level at best: residual 4096 x 4096 23.4 and 26.3
+// against 22.7 us, plain 4096 x 8192 23.4 and 28.3 against 23.7 us; plain rows
+// add in its order from 16 all the same. Rows of 32 KiB of input (residual
+// 8192, plain and residual 16384), and two packets per lane at any width, were
+// 3-18% slower pipelined.
+//
+inline NormRoute norm_route(const NormCall& a, const NormKeys& k) {
+  const bool forced_shape = k.waves_per_row > 0 || k.vecs_per_thread > 0;
+  if (a.nvec <= kShortPackets && !forced_shape && k.force_stream == 0) return {NormKernel::kShort, {0, 0}, 1};
+  if (k.force_stream != 0 || a.nvec > kMaxRegPackets) return {NormKernel::kStream, {0, 0}, 1};
+
+  const bool few = a.rows <= kFewRows;
+  const bool pipe_rows = !few && a.rows < (int64_t(1) << 31) && a.full;
+  const bool pipe_width = (a.nvec == 512 || a.nvec == 1024) && a.row_bytes * (a.residual ? 2 : 1) <= kPipeMaxRowBytes;
+  int64_t rows_per_block = 0;
+  if (k.pipeline == 0 && !forced_shape && pipe_rows && pipe_width)
+    rows_per_block = a.rows / pipe_blocks(static_cast<int>(a.nvec / 64), a.residual, a.rows, a.cus, k.pipe_blocks_per_cu);
+  if (rows_per_block >= kPipeMinRowsPerBlock) return {NormKernel::kPipe, {static_cast<int>(a.nvec / 64), 1}, 1};
+
+  // A plain launch that adds in the pipelined kernel's order without taking it
+  // keeps the shape of large launches.
+  const bool pipe_order = !a.residual && rows_per_block >= kPipeOrderRowsPerBlock;
+  const RegShape order = sum_order(a.nvec, a.residual || few || pipe_order);
+  RegShape s = pipe_order ? sum_order(a.nvec, false) : order;
+  const bool variant_key = k.pipeline == 2 && a.residual;
+  if (!few && !pipe_order && !variant_key && !forced_shape) {
+    const RegShape r = resident_shape(order, a.nvec, a.residual, a.rows);
+    if (r.wpr > 0) s = r;
+  }
+  int sums = order.wpr / s.wpr;
+  if (forced_shape) {
+    const RegShape want{k.waves_per_row > 0 ? k.waves_per_row : s.wpr, k.vecs_per_thread > 0 ? k.vecs_per_thread : s.vpt};
+    for (const RegShape& c : kRegShapes)
+      if (c.wpr == want.wpr && c.vpt == want.vpt && int64_t(c.wpr) * 64 * c.vpt >= a.nvec) s = c;
+    sums = 1;
+  }
+  if (k.pipeline == 2 && pipe_rows && int64_t(s.wpr) * 64 * s.vpt == a.nvec && pipe_shape(s))
+    return {NormKernel::kPipe, s, 1};
+  return {NormKernel::kReg, s, sums};
+}
+
+}  // namespace ako
