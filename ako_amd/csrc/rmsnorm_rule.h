@@ -175,6 +175,9 @@ struct NormRoute {
 // 8192, plain and residual 16384), and two packets per lane at any width, were
 // 3-18% slower pipelined.
 //
+//
+// Resident shapes are for the defaults: a key that names a variant of the
+// large launches' shapes (8 = 2, 9 = 2, 11, 12) gets the shape it belongs to.
 inline NormRoute norm_route(const NormCall& a, const NormKeys& k) {
   const bool forced_shape = k.waves_per_row > 0 || k.vecs_per_thread > 0;
   if (a.nvec <= kShortPackets && !forced_shape && k.force_stream == 0) return {NormKernel::kShort, {0, 0}, 1};
@@ -193,7 +196,7 @@ inline NormRoute norm_route(const NormCall& a, const NormKeys& k) {
   const bool pipe_order = !a.residual && rows_per_block >= kPipeOrderRowsPerBlock;
   const RegShape order = sum_order(a.nvec, a.residual || few || pipe_order);
   RegShape s = pipe_order ? sum_order(a.nvec, false) : order;
-  const bool variant_key = k.pipeline == 2 && a.residual;
+  const bool variant_key = k.early_weights == 2 || k.pipeline == 2 || k.load_groups != 0 || k.write_through != 0;
   if (!few && !pipe_order && !variant_key && !forced_shape) {
     const RegShape r = resident_shape(order, a.nvec, a.residual, a.rows);
     if (r.wpr > 0) s = r;
