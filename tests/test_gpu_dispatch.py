@@ -81,10 +81,11 @@ def test_hip_graph_replays_match_eager() -> None:
     k = _rand(1, 1, 8, 128, seed=4)
     cos, sin = build_rope_tables(1, 128, device=DEV)
     g, u = _rand(1, 14336, seed=5), _rand(1, 14336, seed=6)
-    # Launches of many rows: the persistent pipelined kernel (4096-wide rows)
-    # and bf16 residual rows of 16384 with one-packet load groups.
-    xp, rp = _rand(9000, 4096, seed=7), _rand(9000, 4096, seed=8)
-    xb, rb = _rand(300, 16384, seed=9), _rand(300, 16384, seed=10)
+    # Launches of many rows: the persistent pipelined kernel (4096-wide rows),
+    # a resident shape with separate sums (300 rows of 16384) and the
+    # write-through stores with one-packet load groups (2051).
+    xp, rp = _rand(10300, 4096, seed=7), _rand(10300, 4096, seed=8)
+    xb, rb = _rand(2051, 16384, seed=9), _rand(2051, 16384, seed=10)
     wb = _rand(16384, seed=11, scale=0.1, shift=1.0)
 
     def step():
@@ -96,7 +97,8 @@ def test_hip_graph_replays_match_eager() -> None:
         i = rmsnorm_hip(xp, w)
         j, m = rmsnorm_residual_hip(xp, rp, w)
         n, o = rmsnorm_residual_hip(xb, rb, wb)
-        return a, b, c, d, e, f, h, i, j, m, n, o
+        p, s = rmsnorm_residual_hip(xb[:300], rb[:300], wb)
+        return a, b, c, d, e, f, h, i, j, m, n, o, p, s
 
     eager = step()
     side = torch.cuda.Stream()

@@ -113,7 +113,7 @@ def test_rmsnorm_residual_config2(rows: int, hidden: int, dtype: torch.dtype) ->
 @pytest.mark.parametrize("shape", [(2, 128, 1024), (2, 128, 512), (1, 2048, 4096), (3, 100),
                                    (2, 8448), (5, 1), (4, 7), (3, 65_536), (2, 65_544), (2, 140_000), (1, 262_144)])
 def test_rmsnorm_shapes_dtypes(shape, dtype: torch.dtype) -> None:
-    """Reference test shapes, ragged widths (scalar path), rows wider than the
+    """Reference test shapes, ragged widths, rows wider than the
     register budget (two-pass path), every dtype."""
     x = grandn(shape, dtype, 3, scale=3.0)
     w = grandn(shape[-1:], dtype, 4, scale=0.1, shift=1.0)
@@ -135,11 +135,11 @@ def test_rmsnorm_fp32_weight_and_strided_rows(dtype: torch.dtype) -> None:
     y = rmsnorm_hip(x, w)
     expected = oracle.rmsnorm(to_np(x), to_np(w), dtype=NAMES[dtype], w_dtype="float32")
     assert_oracle(expected, to_np(y), dtype)
-    # Padded stride but a width that is not a multiple of the packet: scalar tail lanes.
+    # Padded stride but a width that is not a multiple of the packet: a partial packet.
     xt = base[:, :4093]
     wt = grandn((4093,), dtype, 8, scale=0.1, shift=1.0)
     assert_oracle(oracle.rmsnorm(to_np(xt), to_np(wt), dtype=NAMES[dtype]), to_np(rmsnorm_hip(xt, wt)), dtype)
-    # Misaligned start (offset by one element): the scalar path.
+    # Misaligned start (offset by one element).
     xm = base.reshape(-1)[1: 1 + 8 * 4096].view(8, 4096)
     assert_oracle(oracle.rmsnorm(to_np(xm), to_np(w), dtype=NAMES[dtype], w_dtype="float32"),
                   to_np(rmsnorm_hip(xm, w)), dtype)
@@ -211,15 +211,16 @@ def test_rmsnorm_xcd_row_orders_cover_every_row(rows: int) -> None:
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("rows", [31, 33, 127, 130, 257, 1000, 2051])
+@pytest.mark.parametrize("rows", [31, 33, 127, 130, 257, 1000, 1603, 2051])
 def test_rmsnorm_wide_rows_xcd_runs_cover_every_row(rows: int, dtype: torch.dtype) -> None:
     """Rows of 16384 half elements go to the XCDs in runs: residual rows in
     runs of 16 from 128 workgroups up (runs of 8 from 64, block order below),
-    plain rows in runs of 4 from 32 workgroups up (block order below). Row
-    counts straddle those thresholds and the 256-row switch to write-through
-    stores, and 1000 / 2051 leave partial runs and trailing blocks; the
-    default order must give bit-identical outputs to block order, which is
-    checked against the oracle on the first and last rows."""
+    plain rows in runs of 4 from 32 workgroups up (block order below), with
+    write-through stores above the resident shapes (1603 and 2051 rows); the
+    resident shapes (257 and 1000 rows) take runs of 8. Row counts straddle
+    those thresholds, and the last three leave partial runs and trailing
+    blocks; the default order must give bit-identical outputs to block order,
+    which is checked against the oracle on the first and last rows."""
     from ako_amd import _native
 
     x = grandn((rows, 16384), dtype, 40)
@@ -272,12 +273,14 @@ def test_rmsnorm_split_launches_match_one_launch(cap: int) -> None:
         _native.set_tuning(0, 9, 0)
 
 
-@pytest.mark.parametrize("hidden,rows", [(4096, 9000), (8192, 4100), (16384, 300)])
+@pytest.mark.parametrize("hidden,rows", [(4096, 9000), (8192, 4100), (16384, 300), (4096, 10300), (8192, 5200),
+                                         (16384, 2051)])
 def test_rmsnorm_padded_output_strides_through_the_abi(hidden, rows) -> None:
-    """Outputs with padded row strides, through the C ABI, at launch sizes the
-    pipelined kernel (4096 and 8192) and the one-packet load groups (bf16
-    16384) take: the padding is never written and the rows equal the
-    contiguous result."""
+    """Outputs with padded row strides, through the C ABI: the padding is never
+    written and the rows equal the contiguous result. The last three are launch
+    sizes that the pipelined kernel (plain 4096 and 8192, residual 4096) and the
+    write-through stores with one-packet load groups (16384) take; 16384 x 300
+    takes a resident shape, the rest the register kernel's large shapes."""
     from ako_amd import _native
 
     lib = _native.load()
@@ -308,13 +311,14 @@ def test_rmsnorm_padded_output_strides_through_the_abi(hidden, rows) -> None:
 def test_rmsnorm_residual_load_groups_match(dtype, w_dtype) -> None:
     """The residual (16 wavefronts, 2 packets) rows with both packets loaded
     as one group (key 11 = 1) and one packet at a time (key 11 = 2): the same
-    sums in the same order, so bit-identical outputs, at a decode-sized and a
-    many-row launch; the default choice against the oracle."""
+    sums in the same order, so bit-identical outputs, at a decode-sized and
+    many-row launches; the default choice (at 300 rows another shape with the
+    same order of sums) against the oracle on sampled rows."""
     from ako_amd import _native
 
     h = 16384
     try:
-        for rows in (33, 300):
+        for rows in (33, 300, 2051):
             x = grandn((rows, h), dtype, 60 + rows)
             r = grandn((rows, h), dtype, 61 + rows)
             w = grandn((h,), w_dtype, 62, scale=0.1, shift=1.0)
@@ -324,9 +328,11 @@ def test_rmsnorm_residual_load_groups_match(dtype, w_dtype) -> None:
                 outs[key] = rmsnorm_residual_hip(x, r, w)
             assert all(torch.equal(a, b) for a, b in zip(outs[1], outs[2])), rows
             assert all(torch.equal(a, b) for a, b in zip(outs[0], outs[1])), rows
-            ey, es = oracle.rmsnorm_residual(to_np(x), to_np(r), to_np(w), dtype=NAMES[dtype], w_dtype=NAMES[w_dtype])
-            np.testing.assert_array_equal(to_np(outs[0][1]), es)
-            assert_oracle(ey, to_np(outs[0][0]), dtype)
+            sel = torch.as_tensor(sample_rows(rows, 300), device=DEV)
+            ey, es = oracle.rmsnorm_residual(to_np(x[sel]), to_np(r[sel]), to_np(w), dtype=NAMES[dtype],
+                                             w_dtype=NAMES[w_dtype])
+            np.testing.assert_array_equal(to_np(outs[0][1][sel]), es)
+            assert_oracle(ey, to_np(outs[0][0][sel]), dtype)
     finally:
         _native.set_tuning(0, 11, 0)
 
@@ -432,12 +438,11 @@ def test_rmsnorm_pipelined_kernel_matches_register_kernel(dtype, w_dtype, hidden
                 assert_oracle(oracle.rmsnorm(to_np(x), to_np(w), dtype=NAMES[dtype], w_dtype=NAMES[w_dtype]),
                               to_np(want_p), dtype)
             # The default choice. Rows of 512 or 1024 packets go pipelined at
-            # one packet per lane (when their input fits 16 KiB; plain rows
-            # only with 16 rows per workgroup, as at 16384 rows) or to the
-            # register kernel's one-packet residual shape: either way the
-            # register kernel at (packets / 64, 1) sums in the same order.
-            # Plain rows short of the row count take the register kernel's
-            # own default shape.
+            # one packet per lane (when their input fits 16 KiB, from 20 rows
+            # per workgroup, as at 16384 rows) or to a register shape. Residual
+            # rows add in the order of the register kernel at (packets / 64, 1)
+            # either way, plain rows from 16 rows per workgroup; below, plain
+            # rows add as the register kernel's own default shape.
             nvec = hidden * x.element_size() // 16
             if shape is None and nvec in (512, 1024):
                 _native.set_tuning(0, 1, nvec // 64)
@@ -578,7 +583,7 @@ def test_rope_config3(batch: int, seq: int, dtype, table_dtype, style: str) -> N
 @pytest.mark.parametrize("shape", [(2, 128, 8, 64), (1, 2048, 32, 128), (2, 6, 3, 8),
                                    (2, 5, 3, 6), (1, 9, 4, 96), (3, 4, 2, 256), (1, 1025, 12, 96)])
 def test_rope_shapes(shape, style: str, dtype) -> None:
-    """Reference test shapes plus head dims on the scalar path (6) and odd packet counts (96);
+    """Reference test shapes plus head dims of less than a packet (6) and odd packet counts (96);
     (1, 1025, 12, 96) is a four-wavefront-workgroup launch whose last workgroup holds
     two spare wavefronts, with idle lanes in every wavefront."""
     x = grandn(shape, dtype, 12)
@@ -614,7 +619,7 @@ def test_rope_strided_views(style: str) -> None:
 CACHE_CASES = [
     (1, 1, 32, 32, 128, 511, 640),  # configs[4] decode step: MHA, slot 511 of 640
     (2, 5, 8, 2, 128, 3, 16),       # GQA, several tokens at once
-    (1, 4, 4, 4, 6, 0, 8),          # head_dim 6: the scalar kernel
+    (1, 4, 4, 4, 6, 0, 8),          # head_dim 6: halves of less than a packet
     (1, 3, 2, 2, 64, 6, 8),         # the last token's slot (8) is past the cache: dropped
     (1, 512, 32, 32, 128, 0, 640),  # configs[4] prefill: 6144 wavefronts, four per workgroup
     (2, 300, 32, 8, 128, 20, 310),  # GQA prefill at an offset, the last 10 tokens past the cache
@@ -686,8 +691,8 @@ def test_rope_every_iteration_count() -> None:
 
 def test_rope_xcd_runs_cover_every_head() -> None:
     """RoPE with workgroups handed to the XCDs in runs (key 3; by default
-    runs of 128 for one tensor from 8192 workgroups, as configs[2]'s q alone
-    at (4, 2048) takes, checked against the oracle in test_rope_config3): the
+    runs of 32 for one tensor from 4096 workgroups, as q alone at (4, 2048, 32,
+    128) takes, checked against the oracle in test_rope_config3): the
     map is a bijection on the grid, so every run length, including ones that
     leave a partial last round and trailing blocks, gives the oracle's exact
     output, for q alone and for q and k in one launch."""
@@ -776,7 +781,7 @@ def test_swiglu_extremes_and_strides(dtype) -> None:
     base_u = grandn((16, 4096 + 8), dtype, 19)
     gs, us = base_g[:, :4096], base_u[:, 8:]
     assert_oracle(oracle.swiglu(to_np(gs), to_np(us), dtype=NAMES[dtype]), to_np(swiglu_hip(gs, us)), dtype)
-    gm = base_g.reshape(-1)[1:1 + 4096 * 3].view(3, 4096)  # misaligned: scalar path
+    gm = base_g.reshape(-1)[1:1 + 4096 * 3].view(3, 4096)  # misaligned
     um = base_u.reshape(-1)[3:3 + 4096 * 3].view(3, 4096)
     assert_oracle(oracle.swiglu(to_np(gm), to_np(um), dtype=NAMES[dtype]), to_np(swiglu_hip(gm, um)), dtype)
     empty = torch.empty(0, 14336, device=DEV, dtype=dtype)

@@ -113,3 +113,34 @@ def test_resident_shapes_hold_no_more_than_a_row(route) -> None:
     launches = [(rows, packets * 8, 2, residual, {}) for packets in WIDTHS for rows in ROWS for residual in (False, True)]
     for (rows, hidden, *_), (_, wpr, vpt, _) in zip(launches, route(launches)):
         assert wpr * vpt * 64 < 2 * (hidden // 8) or wpr * vpt <= 2, (rows, hidden, wpr, vpt)
+
+
+def test_keys_of_a_shape_get_that_shape(route) -> None:
+    """A key that names a variant of the large launches' shapes runs on them at every size above decode."""
+    for keys in ({"load_groups": 1}, {"load_groups": 2}, {"write_through": 1}, {"write_through": 2}):
+        assert route([(300, 16384, 2, res, keys) for res in (False, True)]) == [("reg", 16, 2, 1)] * 2
+    full = [(rows, hidden, 2, res) for rows in (257, 1031, 4099) for hidden in (4096, 8192, 16384, 32768)
+            for res in (False, True)]
+    got = route([(*launch, {"pipeline": 2}) for launch in full])
+    assert {kernel for kernel, *_ in got} == {"pipe"}
+    assert [shape[1:3] for shape in got] == [
+        {4096: (8, 1) if res else (4, 2), 8192: (16, 1) if res else (8, 2), 16384: (16, 2), 32768: (16, 4)}[hidden]
+        for _, hidden, _, res in full]
+
+
+def test_launches_that_the_gpu_tests_name(route) -> None:
+    """The sizes at which GPU tests mean a certain kernel reach it (half elements)."""
+    def kernels(*launches):
+        return route([(rows, hidden, 2, res, {}) for rows, hidden, res in launches])
+
+    # Padded outputs, unaligned rows and captured launches: pipelined, and write-through (16, 2) rows.
+    assert {k for k, *_ in kernels((10300, 4096, False), (10300, 4096, True), (5200, 8192, False))} == {"pipe"}
+    assert kernels((2051, 16384, False), (2051, 16384, True), (1603, 16384, False), (1603, 16384, True)) == [
+        ("reg", 16, 2, 1)] * 4
+    # Resident shapes with separate sums beside them.
+    assert kernels((300, 16384, False), (300, 16384, True), (1000, 16384, False), (1000, 16384, True)) == [
+        ("reg", 8, 4, 2), ("reg", 8, 4, 2), ("reg", 4, 8, 4), ("reg", 8, 4, 2)]
+    # Rows that add in the pipelined kernel's order without taking it.
+    assert kernels((9000, 4096, False), (4100, 8192, False)) == [("reg", 4, 2, 2), ("reg", 8, 2, 2)]
+    assert kernels((9000, 4096, True), (4100, 8192, True)) == [("pipe", 8, 1, 1), ("reg", 16, 1, 1)]
+    assert kernels((2, 70001, False), (2, 70001, True)) == [("stream", 0, 0, 1)] * 2

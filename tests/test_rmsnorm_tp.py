@@ -87,7 +87,7 @@ def test_hip_slices_compose_to_the_full_row(rows: int, hidden: int, shards: int,
     """configs[1] rows and widths cut into 1, 2 or 8 slices (TP=8 puts 2048 of
     16384 on a rank); 4097 rows leave the apply kernel's last workgroup (two
     rows each from 4096 rows on) one row; 4100/2 slices are not 16-byte
-    aligned (scalar path)."""
+    aligned."""
     dev = "cuda"
     x, r = drandn((rows, hidden), dtype, 4), drandn((rows, hidden), dtype, 5)
     w = drandn((hidden,), dtype, 6, scale=0.1, shift=1.0)

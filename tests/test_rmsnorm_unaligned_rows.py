@@ -16,8 +16,8 @@ DEV = "cuda"
 # (rows, hidden): short rows, register rows with and without a partial packet
 # (early and late weights, one and several packets per lane, the shapes whose
 # aligned rows store write-through), the pipelined launches, the two-pass kernel.
-SHAPES = [(5, 3), (33, 80), (3, 515), (40, 4096), (257, 4099), (300, 4096), (9000, 4096), (270, 8191), (300, 16384),
-          (2, 70001)]
+SHAPES = [(5, 3), (33, 80), (3, 515), (40, 4096), (257, 4099), (300, 4096), (10300, 4096), (270, 8191), (300, 16384),
+          (2051, 16384), (2, 70001)]
 
 
 def _rows(rows: int, hidden: int, dtype: torch.dtype, seed: int, start: int, pad: int) -> torch.Tensor:
