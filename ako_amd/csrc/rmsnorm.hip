@@ -242,7 +242,7 @@ __global__ __launch_bounds__(kWave* WPR* RPB) void rmsnorm_reg(
       total += partial[row_in_block][j];
       // Eight sums in registers at a time: sixteen took shapes of eight packets
       // per lane past 80 VGPRs, from 6 wavefronts per SIMD to 5, and launches
-      // that fit at 6 into a second round (bf16, cold, 1500 x 10240 12.5 -> 15.2 us).
+      // that fit at 6 into a second round (bf16, cold, 1500 x 10240 12.8 -> 15.2 us).
       if constexpr (VPT == 8 && SUMS > 1) {
         if (j % 8 == 7) asm volatile("" : "+v"(total) : : "memory");
       }

@@ -78,32 +78,46 @@ inline RegShape sum_order(int64_t nvec, bool one_packet) {
 
 // Shape of a launch of kFewRows to some thousand rows: the one whose wavefronts
 // are resident all at once, so that every row's loads go out at the start and
-// no second round of workgroups waits for the first (a CU holds 32 wavefronts,
-// 24 at eight packets per lane: 8192 and 6144 on the chip). Fewer packets per
-// lane spread a row's latency over more lanes, so the smallest packet count
-// that fits and adds in the row's order is taken, and never 16 wavefronts of
-// more than one packet (plain rows of 10240-16384, 279-500 rows: 10-25% behind
-// 8 of four). Limits from a sweep of every shape over 13 widths x 11 row
-// counts (bf16, cold, MI355X). E.g. against the many-row shapes: residual 512 x
-// 4096 5.6 -> 4.5 us, 2048 x 4096 14.2 -> 12.0, 4096 x 4096 26.6 -> 22.7, 1024 x
-// 8192 14.1 -> 11.9, 1536 x 5120 12.8 -> 11.8; plain 4096 x 3072 11.0 -> 9.1,
-// 1024 x 16384 14.6 -> 12.1.
-struct ResidentLimit {
-  int vpt;
-  int64_t plain_waves, residual_waves;
-};
-constexpr ResidentLimit kResidentLimits[] = {{1, 5120, 5632}, {2, 8192, 4096}, {4, 6144, 8192}, {8, 6144, 0}};
+// no second round of workgroups waits for the first. Fewer packets per lane
+// spread a row's latency over more lanes, so the smallest packet count that
+// fits and adds in the row's order is taken, and never 16 wavefronts of more
+// than one packet (plain rows of 10240-16384, 279-500 rows: 10-25% behind 8 of
+// four). Against the order's own shape, fp16, cold and graph-replayed:
+// residual 512 x 4096 5.8 -> 4.6 us, 2048 x 4096 15.2 -> 12.6, 4096 x 4096 29.5 ->
+// 25.2, 1024 x 8192 15.2 -> 12.8; plain 4096 x 3072 11.9 -> 10.2, 4096 x 4096
+// 14.6 -> 12.8, 1024 x 16384 15.0 -> 13.4.
+//
+// Wavefronts that fit, from sweeps of every shape over 13 widths x 24 row
+// counts (bf16, cold, MI355X). A CU holds 32, 24 at eight packets per lane, but
+// the lead ends earlier where a row's wavefronts come in large workgroups or
+// use most of their packets: past the counts below the next shape is level or
+// up to 15% faster.
+inline int64_t resident_waves(RegShape s, int64_t nvec, bool residual) {
+  if (residual) {
+    // Wavefronts that hold a packet; rows with idle ones last a little longer
+    // (512 x 6144 5.9 us against 6.4 as (8, 2), but full 384 x 8192 8.0 and 7.6).
+    if (s.vpt == 1) return nvec > 64 * (s.wpr - 1) ? 5632 : 6400;
+    // 2400 x 2048 8.9 us against 9.9 as (1, 4), 1200 x 4096 8.9 and 10.1 as (2, 4).
+    if (s.vpt == 2) return 5120;
+    return s.vpt == 4 ? 8192 : 0;
+  }
+  if (s.vpt == 1) return 5120;
+  if (s.vpt == 2) return 8192;
+  // 600 x 14336 10.4 us against 8.5 as (4, 8), but 600 x 10240 6.5 and 7.2.
+  if (s.vpt == 4) return s.wpr == 8 && nvec > 1280 ? 4096 : 6144;
+  // 2100 x 8192 17.1 us against 15.1 as (8, 2), but 2400 x 7168 14.2 and 15.7.
+  return s.wpr == 2 && nvec > 896 ? 4096 : 6144;
+}
 
-// A shape of kResidentLimits that adds in `order`, or {0, 0}. Such a shape
-// holds as many packets over fewer wavefronts, with more sums per lane.
+// A shape whose wavefronts fit and that adds in `order`, or {0, 0}. It holds as
+// many packets over fewer wavefronts, with more sums per lane.
 inline RegShape resident_shape(RegShape order, int64_t nvec, bool residual, int64_t rows) {
   const int total = order.wpr * order.vpt;
-  for (const ResidentLimit& l : kResidentLimits) {
-    const int wpr = total / l.vpt;
-    if (wpr < 1 || wpr > order.wpr || wpr > (l.vpt == 1 ? 16 : 8)) continue;
-    // One packet per lane of residual rows: the wavefronts that hold a packet.
-    const int64_t waves = residual && l.vpt == 1 ? (nvec + 63) / 64 : wpr;
-    if (rows * waves <= (residual ? l.residual_waves : l.plain_waves)) return {wpr, l.vpt};
+  for (int vpt = 1; vpt <= 8; vpt *= 2) {
+    const RegShape s{total / vpt, vpt};
+    if (s.wpr < 1 || s.wpr > order.wpr || s.wpr > (vpt == 1 ? 16 : 8)) continue;
+    const int64_t waves = residual && vpt == 1 ? (nvec + 63) / 64 : s.wpr;
+    if (rows * waves <= resident_waves(s, nvec, residual)) return s;
   }
   return {0, 0};
 }

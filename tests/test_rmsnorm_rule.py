@@ -82,7 +82,7 @@ def _expected_order(packets: int, one_packet: bool) -> int:
 
 WIDTHS = [65, 100, 127, 128, 129, 200, 255, 256, 257, 300, 384, 511, 512, 513, 640, 1000, 1023, 1024, 1025, 1500, 2047,
           2048, 2049, 3000, 4095, 4096, 4097, 6000, 8192]
-ROWS = sorted({1, 2, 255, 256, 257, 100_000} | {limit // waves + off for limit in (4096, 5120, 5632, 6144, 8192, 10240)
+ROWS = sorted({1, 2, 255, 256, 257, 100_000} | {limit // waves + off for limit in (4096, 5120, 5632, 6144, 6400, 7168, 8192, 10240)
                                                 for waves in range(1, 17) for off in (-1, 0, 1)})
 
 
