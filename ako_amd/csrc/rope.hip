@@ -295,8 +295,11 @@ hipError_t run_layout(RopeDev d, int64_t tokens, hipStream_t stream) {
 //   up to 1024: whole heads. One wavefront's latency is the launch's, and one
 //     packet to store is less of it than two: heads of 128, 64 tokens 2.20
 //     against 2.32 us in halves, heads of 80 2.16 against 2.28.
-//   halves of whole 128-byte lines (fp32: of a line or more) above that:
-//     kHalves. 4 x 2048 tokens of heads of 128 27.7 against 29.1 us.
+//   halves of whole 128-byte lines (fp32 and into the caches: of a line or more)
+//     above that: kHalves. 4 x 2048 tokens of heads of 128 27.7 against 29.1 us;
+//     into the caches 48 heads of 192, 512 / 2048 / 4 x 2048 tokens 6.2 / 15.6 /
+//     52.7 against 6.9 / 17.6 / 64.0 us (source rows from memory 6.4 / 16.9 / 55.0
+//     against 6.9 / 20.0 / 66.6).
 //   shorter halves: whole heads, but halves from 2048 to 8192 wavefronts, where
 //     the launch is resident at once and the doubled source and table reads of
 //     whole heads are not hidden: 512 tokens of heads of 64 / 80 / 96 2.74 / 3.17
@@ -304,8 +307,11 @@ hipError_t run_layout(RopeDev d, int64_t tokens, hipStream_t stream) {
 //     5.8 / 6.9 / 7.8 us.
 //   above 16384 wavefronts whole heads of more than a 128-byte line load
 //     without the non-temporal hint, which keeps the lines for the partner
-//     reads: 4 x 2048 tokens of heads of 80 / 96 18.9 / 22.2 against 20.2 / 23.6
-//     us; shorter heads and launches were level or slower.
+//     reads. That is for source rows that the projection before has just
+//     written, still in the MALL: q and k of 40 heads of 80 / 96 / 192, 4 x 2048
+//     tokens 18.1 / 20.9 / 43.3 against 23.2 / 26.9 / 44.1 us in halves. Source
+//     rows from memory are slower so (27.0 / 29.9 / 49.6 against 25.2 / 29.0 /
+//     45.5 us), and so are shorter heads and launches.
 //
 // Against one wavefront per (token, group of heads) in halves for every shape:
 // heads of 64 / 80 / 96 at 4 x 2048 17.6 / 22.4 / 25.9 -> 15.8 / 18.9 / 22.2 us;
@@ -325,7 +331,7 @@ hipError_t run_packet(RopeDev d, bool neox, int64_t tokens, hipStream_t stream) 
   d.last = d.half - E;
   const int64_t packets = ceil_div(d.half, E), half_bytes = d.half * static_cast<int64_t>(sizeof(T));
   const int64_t waves = ceil_div(tokens * d.heads * 2 * packets, kWave);
-  const bool lines = half_bytes >= 128 && (half_bytes % 128 == 0 || sizeof(T) == 4);
+  const bool lines = half_bytes >= 128 && (half_bytes % 128 == 0 || sizeof(T) == 4 || CACHE);
   // kHalves needs a half's packets within one wavefront.
   const bool halves = packets <= kWave && waves > kWholeAlwaysWaves &&
                       (lines || (waves > kHalvesMinWaves && waves <= kHalvesMaxWaves));

@@ -72,7 +72,7 @@ def test_launch_sizes_match_small_launches(head_dim: int, dtype, style: str) -> 
 
 @pytest.mark.parametrize("style", ["neox", "interleaved"])
 @pytest.mark.parametrize("head_dim,dtype", [(6, torch.float32), (72, torch.float16), (80, torch.bfloat16),
-                                            (128, torch.float16)])
+                                            (128, torch.float16), (136, torch.float16), (192, torch.bfloat16)])
 @pytest.mark.parametrize("seq", [1, 700, 4000])
 def test_cache_writes_match_separate_calls(seq: int, head_dim: int, dtype, style: str) -> None:
     """The rotated keys and the values in their slots, every other slot untouched, at each layout's sizes."""
