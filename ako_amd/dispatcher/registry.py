@@ -37,6 +37,8 @@ class KernelRegistry:
 
     def __init__(self) -> None:
         self._by_op: dict[str, list[KernelEntry]] = {}
+        #: Counts the changes, so that a lookup kept elsewhere can tell that it is old.
+        self.generation = 0
 
     def register(self, entry: KernelEntry) -> None:
         """Insert ``entry``; an entry of the same operation and name is replaced."""
@@ -44,12 +46,14 @@ class KernelRegistry:
         kept.append(entry)
         # sorted() is stable: equal priorities keep their registration order.
         self._by_op[entry.op_name] = sorted(kept, key=lambda e: -e.priority)
+        self.generation += 1
 
     def unregister(self, op_name: str, kernel_name: str) -> bool:
         """Drop one kernel; returns whether it was present."""
         entries = self._by_op.get(op_name, [])
         kept = [e for e in entries if e.kernel_name != kernel_name]
         self._by_op[op_name] = kept
+        self.generation += 1
         return len(kept) != len(entries)
 
     def list_ops(self) -> list[str]:

@@ -152,6 +152,7 @@ class KernelSelector:
         self.warmup = warmup
         self.repeats = repeats
         self._memo: dict[tuple[Any, ...], KernelFn] = {}
+        self._forced: dict[tuple[str, str], tuple[int, KernelFn]] = {}
 
     # -- public API ----------------------------------------------------
     def select(
@@ -165,14 +166,16 @@ class KernelSelector:
     ) -> KernelFn:
         """The callable to run for this call; memoised on cheap hashables."""
         if forced:  # the same kernel whatever the tensors: no need to look at them
-            fn = self._memo.get((op_name, forced))
-            if fn is None:
-                fn = self.select_entry(op_name, x, *args, forced=forced, extra_key=extra_key).entry.fn
-                self._memo[(op_name, forced)] = fn
+            # Kept with the registry's state: a kernel replaced or dropped since is looked up again.
+            generation = self.registry.generation
+            known = self._forced.get((op_name, forced))
+            if known is not None and known[0] == generation:
+                return known[1]
+            fn = self.select_entry(op_name, x, *args, forced=forced, extra_key=extra_key).entry.fn
+            self._forced[(op_name, forced)] = (generation, fn)
             return fn
         memo_key = (
             op_name,
-            forced,
             extra_key,
             x.dtype,
             x.shape,
@@ -181,14 +184,13 @@ class KernelSelector:
         )
         fn = self._memo.get(memo_key)
         if fn is None:
-            fn = self.select_entry(
-                op_name, x, *args, forced=forced, extra_key=extra_key, call_kwargs=call_kwargs
-            ).entry.fn
+            fn = self.select_entry(op_name, x, *args, extra_key=extra_key, call_kwargs=call_kwargs).entry.fn
             self._memo[memo_key] = fn
         return fn
 
     def clear_memo(self) -> None:
         self._memo.clear()
+        self._forced.clear()
 
     def select_entry(
         self,

@@ -1,4 +1,4 @@
-"""A forced kernel is looked up by its name alone, and again after the memo is cleared."""
+"""A forced kernel is looked up by its name alone, and again once the registry changed or the memo is cleared."""
 
 from __future__ import annotations
 
@@ -26,3 +26,19 @@ def test_forced_kernels(tmp_path) -> None:
     registry.register(KernelEntry("op", "b", first, backend="hip", priority=5))
     selector.clear_memo()
     assert selector.select("op", torch.zeros(2), forced="b") is first
+
+
+def test_forced_kernels_follow_the_registry(tmp_path) -> None:
+    """A kernel replaced or dropped after a forced call is not called again, at any shape."""
+    registry = KernelRegistry()
+    first, second = (lambda x: x), (lambda x: x + 1)
+    registry.register(KernelEntry("op", "a", first, backend="pytorch", priority=10))
+    registry.register(KernelEntry("op", "b", first, backend="hip", priority=5))
+    selector = KernelSelector(registry=registry, cache=KernelCache(path=tmp_path / "cache.json"))
+    assert selector.select("op", torch.zeros(2), forced="b") is first
+    registry.register(KernelEntry("op", "b", second, backend="hip", priority=5))
+    assert selector.select("op", torch.zeros(3), forced="b") is second
+    assert selector.select("op", torch.zeros(2), forced="b") is second
+    registry.unregister("op", "b")
+    with pytest.raises(ValueError, match="Unknown kernel"):
+        selector.select("op", torch.zeros(3), forced="b")
