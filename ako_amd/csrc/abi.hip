@@ -185,7 +185,7 @@ int ako_set_tuning(int op, int key, int value) {
       break;
     case 1:
       if (key == 1) { ako::g_rope_tuning.waves_per_block = value; return AKO_OK; }
-      if (key == 2) { ako::g_rope_tuning.iters = value; return AKO_OK; }
+      if (key == 2) return AKO_OK;  // head groups per wavefront, once: every lane moves one packet
       if (key == 3) { ako::g_rope_tuning.xcd_chunk = value; return AKO_OK; }
       break;
     case 2:

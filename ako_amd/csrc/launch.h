@@ -71,12 +71,11 @@ struct RmsTuning {
 };
 struct RopeTuning {
   TuningKey waves_per_block{0};  // key 1: wavefronts per workgroup (1, or 4 for any other value; 0 = by launch size)
-  TuningKey iters{0};            // key 2: accepted and unused (every lane moves one packet)
   TuningKey xcd_chunk{0};        // key 3: consecutive workgroups per XCD run (1 = block order; 0 = by launch)
 };
 struct SwigluTuning {
   TuningKey vecs_per_thread{0};  // key 1: packets per lane (1, 2, 4 or 8)
-  TuningKey xcd_chunk{0};        // key 2: consecutive workgroups per XCD run in dense launches (1 = block order; 0 = runs of 4 for launches of 2048-65535 workgroups)
+  TuningKey xcd_chunk{0};        // key 2: consecutive workgroups per XCD run (1 = block order; 0 = runs of 4 for launches of 2048-65535 workgroups)
 };
 extern RmsTuning g_rms_tuning;
 extern RopeTuning g_rope_tuning;

@@ -675,18 +675,19 @@ def test_rope_qk_cache_without_values_and_rejects() -> None:
         rope_qk_cache_hip(q, k, k, cos, sin, pos, kc, None)
 
 
-def test_rope_every_iteration_count() -> None:
+def test_rope_every_workgroup_size() -> None:
+    """One and four wavefronts per workgroup (key 1), 40 heads, the last workgroup partial."""
     from ako_amd import _native
 
     x = grandn((3, 7, 40, 128), torch.float16, 14)
     cos, sin = build_rope_tables(7, 128, device=DEV)
     expected = oracle.rope(to_np(x), to_np(cos), to_np(sin), "neox", dtype="float16")
     try:
-        for iters in (1, 2, 4, 8):
-            _native.set_tuning(1, 2, iters)
+        for waves in (0, 1, 4):
+            _native.set_tuning(1, 1, waves)
             assert_rope_exact(expected, to_np(rope_hip(x, cos, sin)), torch.float16)
     finally:
-        _native.set_tuning(1, 2, 0)
+        _native.set_tuning(1, 1, 0)
 
 
 def test_rope_xcd_runs_cover_every_head() -> None:

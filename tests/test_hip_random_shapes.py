@@ -126,9 +126,9 @@ def test_rope_random_cases(seed: int) -> None:
         x = full[:, :, 1:h + 1]  # a strided head slice
         cos, sin = build_rope_tables(s, d, offset=offset, device=DEV)
         cos, sin = cos.to(tdtype), sin.to(tdtype)
-        # Wavefronts per workgroup (0: the default); 2-16 leave spare
-        # wavefronts in the last workgroup, which must write nothing.
-        per_block = int(rng.choice([0, 1, 2, 4, 8, 16]))
+        # Wavefronts per workgroup (0: the default); 4 leaves spare wavefronts
+        # in the last workgroup, which must write nothing.
+        per_block = int(rng.choice([0, 1, 4]))
         case = (f"b={b} s={s} h={h} d={d} {style} {dtype} tables {tdtype} offset={offset} "
                 f"waves/workgroup={per_block}")
         try:

@@ -51,7 +51,7 @@ def test_short_rows(dtype, extra: int) -> None:
     per_packet = 16 // dtype.itemsize
     for packets in PACKETS:
         hidden = packets * per_packet + extra
-        if hidden == 0 or (packets == 64 and extra):
+        if hidden == 0:
             continue
         for rows in (1, 3, 33, 259):
             case = f"{rows}x{hidden} {dtype}"
@@ -78,9 +78,8 @@ def test_short_rows_of_many_row_launches(hidden: int, rows: int, dtype) -> None:
     y = rmsnorm_hip(x, w, 1e-6)
     yr, s = rmsnorm_residual_hip(x, r, w, 1e-6)
     assert torch.equal(s, x + r)
-    if x.is_contiguous() or hidden % 8 == 0:  # the register kernel needs aligned rows too
-        assert torch.equal(y, _one_wavefront_per_row(lambda: rmsnorm_hip(x, w, 1e-6)))
-        assert torch.equal(yr, _one_wavefront_per_row(lambda: rmsnorm_residual_hip(x, r, w, 1e-6)[0]))
+    assert torch.equal(y, _one_wavefront_per_row(lambda: rmsnorm_hip(x, w, 1e-6)))
+    assert torch.equal(yr, _one_wavefront_per_row(lambda: rmsnorm_residual_hip(x, r, w, 1e-6)[0]))
     pick = torch.tensor([0, 1, rows // 2, rows - 2, rows - 1], device=DEV)
     rep = oracle.gate(oracle.rmsnorm(to_np(x[pick]), to_np(w), 1e-6, dtype=NAMES[dtype]), to_np(y[pick]), NAMES[dtype])
     assert rep["passed"] and rep["err_ulps"] <= MAX_ULPS[dtype], rep
