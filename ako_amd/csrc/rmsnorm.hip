@@ -1000,16 +1000,11 @@ hipError_t run_shard_partial(const RmsShardArgs& a, hipStream_t stream) {
 
 template <typename T, typename W, int R>
 hipError_t run_shard_apply_r(const RmsShardArgs& a, hipStream_t stream) {
-  const int64_t cap = max_blocks_per_launch(kStreamBlock) * R;  // rows per launch
+  const int64_t blocks = max_blocks_per_launch(kStreamBlock), cap = blocks * R;  // rows per launch
   const float inv_h = 1.0f / static_cast<float>(a.hidden);
   for (int64_t r0 = 0; r0 < a.rows; r0 += cap) {
     const int64_t end = std::min(a.rows, r0 + cap);
-    // Rows a multiple of 8 apart: their workgroup runs on the XCD whose
-    // workgroups of the partial half wrote them (workgroup b runs on XCD b % 8),
-    // and finds what is left of them in its L2 (both halves, outputs over those
-    // of the call before, 4096 rows of 2048: 21.2 us with neighbouring rows,
-    // 15.7 us so).
-    const int64_t apart = R == 1 ? end - r0 : ceil_div(ceil_div(end - r0, R), 8) * 8;
+    const int64_t apart = shard_rows_apart(end - r0, R, blocks);
     const dim3 grid(static_cast<unsigned>(std::min(apart, end - r0)));
     AKO_LAUNCH((rmsnorm_shard_apply<T, W, R>), grid, dim3(kStreamBlock), 0, stream,
                static_cast<const T*>(a.x), static_cast<const W*>(a.w), a.total, static_cast<T*>(a.y), r0, end, apart,

@@ -165,6 +165,20 @@ inline int64_t pipe_blocks(int wpr, bool residual, int64_t rows, int cus, int fo
   return blocks >= 16 ? blocks / 8 * 8 : 8;
 }
 
+// Rows between the rows of one workgroup of rmsnorm_shard_apply, in a launch of
+// `rows` rows, `per_block` to a workgroup, and its workgroups: as many, or the
+// rows if fewer. A multiple of 8: such a row's workgroup runs on the XCD whose
+// workgroups of the partial half wrote it (workgroup b runs on XCD b % 8), and
+// finds what is left of it in its L2 (both halves, outputs over those of the
+// call before, 4096 rows of 2048: 21.2 us with neighbouring rows, 15.7 us so).
+// Never more than `max_blocks`, which holds the launch's rows.
+inline int64_t shard_rows_apart(int64_t rows, int per_block, int64_t max_blocks) {
+  if (per_block == 1) return rows;
+  const int64_t blocks = (rows + per_block - 1) / per_block;
+  const int64_t apart = (blocks + 7) / 8 * 8;
+  return apart < max_blocks ? apart : max_blocks;
+}
+
 enum class NormKernel { kShort, kReg, kPipe, kStream };
 struct NormRoute {
   NormKernel kernel;

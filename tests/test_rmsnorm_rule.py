@@ -21,12 +21,32 @@ CSRC = Path(__file__).resolve().parent.parent / "ako_amd" / "csrc"
 
 DRIVER = r"""
 #include <cstdio>
-#include <cstdlib>
+#include <vector>
 #include "rmsnorm_rule.h"
 using namespace ako;
 
-// rule <nvec> <full> <row bytes> <rows> <residual> <cus> <8 keys>, one launch per input line.
-int main() {
+// Without arguments, norm_route of the launches on stdin:
+// <nvec> <full> <row bytes> <rows> <residual> <cus> <8 keys>, one launch per input line.
+int shards() {  // every row of a launch in one workgroup, and no more workgroups than allowed
+  long bad = 0;
+  for (int64_t cap : {1, 2, 3, 5, 8, 9, 64, 1000})
+    for (int64_t rows = 1; rows <= 2 * cap; ++rows)
+      for (int per_block = 1; per_block <= 2; ++per_block) {
+        if (rows > cap * per_block) continue;
+        const int64_t apart = shard_rows_apart(rows, per_block, cap), blocks = apart < rows ? apart : rows;
+        std::vector<int> taken(rows);
+        for (int64_t b = 0; b < blocks; ++b)
+          for (int64_t r = b, k = 0; k < per_block && r < rows; r += apart, ++k) ++taken[r];
+        bad += blocks > cap;
+        for (int t : taken) bad += t != 1;
+        if (per_block > 1 && cap >= rows + 8) bad += apart % 8 != 0;
+      }
+  std::printf("%ld\n", bad);
+  return bad != 0;
+}
+
+int main(int argc, char**) {
+  if (argc > 1) return shards();
   long long nvec, bytes, rows;
   int full, residual, cus, k[8];
   while (std::scanf("%lld %d %lld %lld %d %d", &nvec, &full, &bytes, &rows, &residual, &cus) == 6) {
@@ -69,7 +89,14 @@ def route(tmp_path_factory):
             assert sums in (1, instantiated), launch  # a launch never asks for a variant that is not compiled
         return [(KERNELS[kernel], wpr, vpt, sums) for kernel, wpr, vpt, sums, _ in values]
 
+    ask.exe = folder / "rule"
     return ask
+
+
+def test_sharded_rows_fill_no_more_workgroups_than_allowed(route) -> None:
+    """Two rows a workgroup, a multiple of 8 apart: each row once, within the cap on workgroups (key 7)."""
+    out = subprocess.run([str(route.exe), "shards"], capture_output=True, text=True, timeout=60)
+    assert out.returncode == 0, out.stdout
 
 
 def _expected_order(packets: int, one_packet: bool) -> int:
