@@ -604,7 +604,8 @@ __global__ __launch_bounds__(kStreamBlock) void rmsnorm_shard_partial(
     }
     ss = sumsq_add(p, ss);
   }
-  for (int j = nvec * E + tid; j < shard; j += kStreamBlock) {  // past the last whole packet
+  if (tid < shard - nvec * E) {  // past the last whole packet (no sum that could pass 2^31 - 1)
+    const int j = nvec * E + tid;
     T v = xr[j];
     if constexpr (RES) {
       v = from_f32<T>(to_f32(v) + to_f32(res[row * sr + j]));
@@ -663,16 +664,14 @@ __global__ __launch_bounds__(kStreamBlock) void rmsnorm_shard_apply(
     for (int k = 0; k < R; ++k)
       if (first + k * apart < rows) apply(first + k * apart, vi, p[k], wf, rstd[k]);
   }
-  const int tail0 = nvec * E + tid;
-  if (tail0 < shard) {
+  if (tid < shard - nvec * E) {
+    const int j = nvec * E + tid;
 #pragma unroll
     for (int k = 0; k < R; ++k) {
       const int64_t row = first + k * apart;
       if (row >= rows) break;
       const float rs = rsqrtf(total[row] * inv_h + eps);
-      const T* sr = s + row * ss_;
-      T* yr = y + row * sy;
-      for (int j = tail0; j < shard; j += kStreamBlock) yr[j] = from_f32<T>((to_f32(sr[j]) * rs) * to_f32(w[j]));
+      y[row * sy + j] = from_f32<T>((to_f32(s[row * ss_ + j]) * rs) * to_f32(w[j]));
     }
   }
 }
