@@ -74,7 +74,7 @@ struct RopeTuning {
   TuningKey xcd_chunk{0};        // key 3: consecutive workgroups per XCD run (1 = block order; 0 = by launch)
 };
 struct SwigluTuning {
-  TuningKey vecs_per_thread{0};  // key 1: packets per lane (1, 2, 4 or 8)
+  TuningKey vecs_per_thread{0};  // key 1: packets per lane of dense launches (1, 2, 4 or 8)
   TuningKey xcd_chunk{0};        // key 2: consecutive workgroups per XCD run (1 = block order; 0 = runs of 4 for launches of 2048-65535 workgroups)
 };
 extern RmsTuning g_rms_tuning;

@@ -203,7 +203,6 @@ struct NormRoute {
 // 8192, plain and residual 16384), and two packets per lane at any width, were
 // 3-18% slower pipelined.
 //
-//
 // Resident shapes are for the defaults: a key that names a variant of the
 // large launches' shapes (8 = 2, 9 = 2, 11, 12) gets the shape it belongs to.
 inline NormRoute norm_route(const NormCall& a, const NormKeys& k) {
