@@ -16,8 +16,9 @@
 //   kWhole        neox: a lane holds one packet of the head and reads the
 //                 partner packet half a head away too, but writes only its
 //                 own, so a wavefront's loads and stores run through whole
-//                 heads. For halves shorter than a 128-byte line, where
-//                 kHalves touches every line in two instructions.
+//                 heads. For small launches, and for halves that are no
+//                 whole lines, whose lines kHalves touches in two
+//                 instructions (run_packet has the sizes).
 //
 // Packets need no alignment (common.h), so any strides and table offsets take
 // them. Where a half (interleaved: a head) is no whole number of packets, the
@@ -75,7 +76,7 @@ struct RopeDev {
 enum RopeLayout { kInterleaved, kHalves, kWhole };
 
 // LNT: non-temporal source loads. kWhole reads every line through two packets
-// of neighbouring lanes and wants it kept for the second.
+// and mostly wants it kept for the second (run_packet).
 template <typename T, typename TT, RopeLayout LAYOUT, int E, bool LNT, bool CACHE, int BLOCK>
 __global__ __launch_bounds__(BLOCK) void rope_packets(RopeDev a) {
   constexpr int NT = LAYOUT == kInterleaved ? E / 2 : E;  // table values per lane
@@ -289,37 +290,46 @@ hipError_t run_layout(RopeDev d, int64_t tokens, hipStream_t stream) {
              : run_block<T, TT, LAYOUT, E, LNT, CACHE, 4 * kWave>(d, units, stream);
 }
 
-// neox layouts, by the wavefronts that whole heads would take and the bytes of
-// a half. Against both others, MI355X, fp16, 40 heads, cold:
+// neox layouts, by the wavefronts (1 KiB of source rows each) that whole heads
+// would take and the bytes of a half. MI355X, fp16, 40 heads; "in cache": source
+// rows that a kernel has just written, as the projection before does, else
+// rows from memory.
 //
 //   up to 1024: whole heads. One wavefront's latency is the launch's, and one
 //     packet to store is less of it than two: heads of 128, 64 tokens 2.20
 //     against 2.32 us in halves, heads of 80 2.16 against 2.28.
-//   halves of whole 128-byte lines (fp32 and into the caches: of a line or more)
-//     above that: kHalves. 4 x 2048 tokens of heads of 128 27.7 against 29.1 us;
-//     into the caches 48 heads of 192, 512 / 2048 / 4 x 2048 tokens 6.2 / 15.6 /
-//     52.7 against 6.9 / 17.6 / 64.0 us (source rows from memory 6.4 / 16.9 / 55.0
-//     against 6.9 / 20.0 / 66.6).
-//   shorter halves: whole heads, but halves from 2048 to 8192 wavefronts, where
-//     the launch is resident at once and the doubled source and table reads of
-//     whole heads are not hidden: 512 tokens of heads of 64 / 80 / 96 2.74 / 3.17
-//     / 3.53 against 2.88 / 3.24 / 3.72 us; 2048 tokens 6.3 / 7.8 / 8.6 against
-//     5.8 / 6.9 / 7.8 us.
-//   above 16384 wavefronts whole heads of more than a 128-byte line load
-//     without the non-temporal hint, which keeps the lines for the partner
-//     reads. That is for source rows that the projection before has just
-//     written, still in the MALL: q and k of 40 heads of 80 / 96 / 192, 4 x 2048
-//     tokens 18.1 / 20.9 / 43.3 against 23.2 / 26.9 / 44.1 us in halves. Source
-//     rows from memory are slower so (27.0 / 29.9 / 49.6 against 25.2 / 29.0 /
-//     45.5 us), and so are shorter heads and launches.
+//   halves of a 128-byte line or more above that: kHalves. 4 x 2048 tokens of
+//     heads of 128 27.7 against 29.1 us; heads of 192, 1024 tokens 7.9 against 8.6
+//     us (in cache 8.6 and 11.0), 8192 tokens 44.7 and 48.5 (35.6 and 38.3); into
+//     the caches, 48 heads of 192, 512 / 2048 / 4 x 2048 tokens 6.2 / 15.6 / 52.7
+//     against 6.9 / 17.6 / 64.0 us.
+//   but whole heads from 16384 to 40960, whose rows stay in the cache between the
+//     projection and this launch, where such halves are no whole lines: in cache
+//     2048 tokens of heads of 160 / 208 10.7 / 13.4 against 11.7 / 13.7 us (from
+//     memory 12.7 / 15.8 and 12.1 / 14.8), and from 16384 on where they are no whole
+//     packets either (heads of 136, 2048 / 4096 tokens in cache 10.4 / 17.0 against
+//     11.4 / 20.3 us, from memory level). Not into the caches, where it is slower.
+//   shorter halves: whole heads, but halves from 2048 to 8192, where the launch
+//     is resident at once and the doubled source and table reads of whole heads
+//     are not hidden: 512 tokens of heads of 64 / 80 / 96 2.74 / 3.17 / 3.53 against
+//     2.88 / 3.24 / 3.72 us; 2048 tokens 6.3 / 7.8 / 8.6 against 5.8 / 6.9 / 7.8 us.
+//
+// Whole heads read every line twice and load without the non-temporal hint,
+// which keeps the lines for the partner reads. In cache, with the hint / without:
+// heads of 72 / 80 / 136, 64 tokens 2.48 / 2.16 / 2.68 -> 2.18 / 1.96 / 2.40 us,
+// heads of 80 / 96, 2048 tokens 10.4 / 10.9 -> 9.1 / 8.8, heads of 80 into the
+// caches, 1536 tokens 10.6 -> 9.9; from memory level (heads of 80 / 96, 2048 tokens
+// 7.7 / 8.6 -> 7.9 / 8.7).
+// Only launches of more than kHalvesMaxWaves of halves of at most 64 bytes have
+// it: there rows from memory lose more (2048 tokens of heads of 64 6.4 -> 6.7 us).
 //
 // Against one wavefront per (token, group of heads) in halves for every shape:
 // heads of 64 / 80 / 96 at 4 x 2048 17.6 / 22.4 / 25.9 -> 15.8 / 18.9 / 22.2 us;
 // heads of 72, one lane per rotated pair then, 61 -> 18.6 us; interleaved heads
-// of 80 / 192 19.4 / 50 -> 18.2 / 40.4 us; heads of 128 unchanged.
+// of 80 / 192 19.4 / 50 -> 18.2 / 40.4 us; heads of 128 and 192 unchanged.
 constexpr int64_t kWholeAlwaysWaves = 1024;
 constexpr int64_t kHalvesMinWaves = 2048, kHalvesMaxWaves = 8192;
-constexpr int64_t kWholeCachedWaves = 16384;
+constexpr int64_t kWholeCachedWaves = 16384, kWholeCachedMaxWaves = 40960;
 
 template <typename T, typename TT, int E, bool CACHE>
 hipError_t run_packet(RopeDev d, bool neox, int64_t tokens, hipStream_t stream) {
@@ -331,14 +341,16 @@ hipError_t run_packet(RopeDev d, bool neox, int64_t tokens, hipStream_t stream) 
   d.last = d.half - E;
   const int64_t packets = ceil_div(d.half, E), half_bytes = d.half * static_cast<int64_t>(sizeof(T));
   const int64_t waves = ceil_div(tokens * d.heads * 2 * packets, kWave);
-  const bool lines = half_bytes >= 128 && (half_bytes % 128 == 0 || sizeof(T) == 4 || CACHE);
+  const bool whole_lines = half_bytes % 128 == 0 || sizeof(T) == 4 || CACHE;
+  const bool whole_cached = !whole_lines && waves > kWholeCachedWaves &&
+                            (waves <= kWholeCachedMaxWaves || half_bytes % 16 != 0);
   // kHalves needs a half's packets within one wavefront.
   const bool halves = packets <= kWave && waves > kWholeAlwaysWaves &&
-                      (lines || (waves > kHalvesMinWaves && waves <= kHalvesMaxWaves));
+                      (half_bytes >= 128 ? !whole_cached : waves > kHalvesMinWaves && waves <= kHalvesMaxWaves);
   if (halves) return run_layout<T, TT, kHalves, E, true, CACHE>(d, tokens, stream);
-  if (waves > kWholeCachedWaves && half_bytes > 64)
-    return run_layout<T, TT, kWhole, E, false, CACHE>(d, tokens, stream);
-  return run_layout<T, TT, kWhole, E, true, CACHE>(d, tokens, stream);
+  if (waves > kHalvesMaxWaves && half_bytes <= 64)
+    return run_layout<T, TT, kWhole, E, true, CACHE>(d, tokens, stream);
+  return run_layout<T, TT, kWhole, E, false, CACHE>(d, tokens, stream);
 }
 
 // Elements per packet: 16 bytes, or the largest smaller power of two that a

@@ -48,12 +48,12 @@ def test_head_dims_match_the_oracle(start: int, dtype, style: str) -> None:
                 np.testing.assert_array_equal(to_np(got), expected, err_msg=f"{head_dim} {tdt}")
 
 
-# Wavefronts of whole 16-byte packets, 12 heads: below 1024, either side of
-# 2048, of 8192 and of 16384.
+# Wavefronts of whole 16-byte packets, 12 heads: either side of 2048 and of
+# 8192, against slices below 1024.
 @pytest.mark.parametrize("style", ["neox", "interleaved"])
 @pytest.mark.parametrize("head_dim,dtype", [(32, torch.float16), (72, torch.bfloat16), (80, torch.float16),
-                                            (128, torch.float16), (160, torch.bfloat16), (72, torch.float32),
-                                            (1042, torch.float16)])
+                                            (128, torch.float16), (160, torch.bfloat16), (192, torch.float16),
+                                            (72, torch.float32), (1042, torch.float16)])
 def test_launch_sizes_match_small_launches(head_dim: int, dtype, style: str) -> None:
     per_token = 12 * head_dim * dtype.itemsize / 1024  # wavefronts
     for waves in (1500, 5000, 12000, 20000):
