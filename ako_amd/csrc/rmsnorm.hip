@@ -629,12 +629,13 @@ __global__ __launch_bounds__(kStreamBlock) void rmsnorm_shard_partial(
 template <typename T, typename W, int R>
 __global__ __launch_bounds__(kStreamBlock) void rmsnorm_shard_apply(
     const T* __restrict__ s, const W* __restrict__ w, const float* __restrict__ total,
-    T* __restrict__ y, int64_t row0, int64_t rows, int64_t apart, int shard, int64_t ss_, int64_t sy, float inv_h, float eps) {
-  // Each workgroup applies R rows `apart` rows from each other; a lane holds the
-  // same columns of all R, so the weight packet is read once for R rows.
+    T* __restrict__ y, int64_t row0, int64_t rows, int shard, int64_t ss_, int64_t sy, float inv_h, float eps) {
+  // Each workgroup applies R rows (8 apart: shard_blocks); a lane holds the same
+  // columns of all R, so the weight packet is read once for R rows.
+  constexpr int64_t apart = 8;
   constexpr int E = 16 / static_cast<int>(sizeof(T));
   using P = Pack<T, E>;
-  const int64_t first = row0 + blockIdx.x;
+  const int64_t first = row0 + (R == 1 ? blockIdx.x : static_cast<int64_t>(blockIdx.x / 8) * (8 * R) + blockIdx.x % 8);
   const int tid = threadIdx.x;
   const int nvec = shard / E;
   const auto apply = [&](int64_t row, int vi, const P& p, const float (&wf)[E], float rstd) {
@@ -999,14 +1000,13 @@ hipError_t run_shard_partial(const RmsShardArgs& a, hipStream_t stream) {
 
 template <typename T, typename W, int R>
 hipError_t run_shard_apply_r(const RmsShardArgs& a, hipStream_t stream) {
-  const int64_t blocks = max_blocks_per_launch(kStreamBlock), cap = blocks * R;  // rows per launch
+  const int64_t cap = shard_launch_rows(R, max_blocks_per_launch(kStreamBlock));
   const float inv_h = 1.0f / static_cast<float>(a.hidden);
   for (int64_t r0 = 0; r0 < a.rows; r0 += cap) {
     const int64_t end = std::min(a.rows, r0 + cap);
-    const int64_t apart = shard_rows_apart(end - r0, R, blocks);
-    const dim3 grid(static_cast<unsigned>(std::min(apart, end - r0)));
+    const dim3 grid(static_cast<unsigned>(shard_blocks(end - r0, R)));
     AKO_LAUNCH((rmsnorm_shard_apply<T, W, R>), grid, dim3(kStreamBlock), 0, stream,
-               static_cast<const T*>(a.x), static_cast<const W*>(a.w), a.total, static_cast<T*>(a.y), r0, end, apart,
+               static_cast<const T*>(a.x), static_cast<const W*>(a.w), a.total, static_cast<T*>(a.y), r0, end,
                static_cast<int>(a.shard), a.sx, a.sy, inv_h, a.eps);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) return err;
@@ -1020,7 +1020,7 @@ hipError_t run_shard_apply_r(const RmsShardArgs& a, hipStream_t stream) {
 // beat one, and four were no faster than two.
 template <typename T, typename W>
 hipError_t run_shard_apply(const RmsShardArgs& a, hipStream_t stream) {
-  if (a.rows >= 4096) return run_shard_apply_r<T, W, 2>(a, stream);
+  if (a.rows >= 4096 && max_blocks_per_launch(kStreamBlock) >= 8) return run_shard_apply_r<T, W, 2>(a, stream);
   return run_shard_apply_r<T, W, 1>(a, stream);
 }
 

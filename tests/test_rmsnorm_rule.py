@@ -29,18 +29,23 @@ using namespace ako;
 // <nvec> <full> <row bytes> <rows> <residual> <cus> <8 keys>, one launch per input line.
 int shards() {  // every row of a launch in one workgroup, and no more workgroups than allowed
   long bad = 0;
-  for (int64_t cap : {1, 2, 3, 5, 8, 9, 64, 1000})
-    for (int64_t rows = 1; rows <= 2 * cap; ++rows)
-      for (int per_block = 1; per_block <= 2; ++per_block) {
-        if (rows > cap * per_block) continue;
-        const int64_t apart = shard_rows_apart(rows, per_block, cap), blocks = apart < rows ? apart : rows;
+  for (int64_t cap : {1, 2, 3, 5, 8, 9, 15, 16, 64, 1000})
+    for (int per_block = 1; per_block <= 2; ++per_block) {
+      const int64_t most = shard_launch_rows(per_block, cap);
+      if (cap >= 8) bad += most <= 0;
+      for (int64_t rows = 1; rows <= most; ++rows) {
+        const int64_t blocks = shard_blocks(rows, per_block);
         std::vector<int> taken(rows);
         for (int64_t b = 0; b < blocks; ++b)
-          for (int64_t r = b, k = 0; k < per_block && r < rows; r += apart, ++k) ++taken[r];
+          for (int64_t k = 0; k < per_block; ++k) {
+            const int64_t r = (per_block == 1 ? b : b / 8 * (8 * per_block) + b % 8) + 8 * k;
+            if (r < rows) ++taken[r];
+            bad += r % 8 != b % 8;  // the XCD that the row was written on
+          }
         bad += blocks > cap;
         for (int t : taken) bad += t != 1;
-        if (per_block > 1 && cap >= rows + 8) bad += apart % 8 != 0;
       }
+    }
   std::printf("%ld\n", bad);
   return bad != 0;
 }
@@ -94,7 +99,7 @@ def route(tmp_path_factory):
 
 
 def test_sharded_rows_fill_no_more_workgroups_than_allowed(route) -> None:
-    """Two rows a workgroup, a multiple of 8 apart: each row once, within the cap on workgroups (key 7)."""
+    """Two rows a workgroup, 8 apart: each row once, on its XCD, within the cap on workgroups (key 7)."""
     out = subprocess.run([str(route.exe), "shards"], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0, out.stdout
 

@@ -1,7 +1,7 @@
 """The apply half of the sharded RMSNorm at the row counts where a workgroup
-takes two rows (4096 up), a multiple of 8 rows apart: even, odd and ragged
-halves, each row the same as in a launch of one row per workgroup; and both
-halves at the widest slice."""
+takes two rows (4096 up), 8 apart: whole and partial groups of 16 rows, each
+row the same as in a launch of one row per workgroup; and both halves at the
+widest slice."""
 
 from __future__ import annotations
 
